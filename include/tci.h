@@ -154,13 +154,15 @@ tci_status tci_rrlu_batched_f64(tci_ctx *ctx, tci_lu_job *jobs_device, int64_t c
  * tci_rrlu_batched_f64) use; no counterpart in the reference, and the results
  * are the same bits either way.  AUTO (the default): the register-tile
  * factorization (one workgroup) for matrices up to 128×128; the cooperative
- * whole-chip factorization (one workgroup per CU) for matrices of at least
- * 384² elements with sides up to 8192 when a batch holds at most 8 of them;
- * the streaming one-workgroup factorization otherwise.  STREAM: always
- * streaming; TILE: always the register tile (jobs larger than 128×128 are
- * refused with TCI_ERR_ARG); GRID: the cooperative factorization for every
- * job with sides up to 8192, one job after the other.  The no-allocation
- * entry below never uses the cooperative kernel. */
+ * on-chip factorization (a team of workgroups holds the matrix in registers,
+ * all jobs of a batch in one launch) for the others with sides up to 8192;
+ * the streaming one-workgroup factorization beyond.  While a slot server is
+ * running on the device the on-chip kernels, whose launch would wait for its
+ * grid to leave, take only jobs of at least 384² elements, when a batch holds
+ * at most 8 of them.  STREAM: always streaming; TILE: always the register
+ * tile (jobs larger than 128×128 are refused with TCI_ERR_ARG); GRID: the
+ * on-chip factorization for every job with sides up to 8192.  The
+ * no-allocation entry below never uses the cooperative kernels. */
 enum { TCI_RRLU_AUTO = 0, TCI_RRLU_STREAM = 1, TCI_RRLU_TILE = 2, TCI_RRLU_GRID = 3 };
 tci_status tci_ctx_set_rrlu_algo(tci_ctx *ctx, int32_t algo);
 
@@ -168,14 +170,14 @@ tci_status tci_ctx_set_rrlu_algo(tci_ctx *ctx, int32_t algo);
  * For square matrices of each bucket side (32, 64, ..., 4096; rank
  * min(side/2, 64), reltol 1e-10) it times on this context's device: the
  * register tile against the streaming kernel for a batch of 512 (sides up
- * to 128), the cooperative kernel at 256, 512 and 1024 threads for one
- * matrix, and k cooperative runs one after the other against one streaming
- * launch of k matrices (k = 1, 2, 4, ..., 64).  The winners are stored in
+ * to 128), the cooperative on-chip kernel for one matrix, and one on-chip
+ * launch of k matrices against one streaming launch of k (k = 1, 2, 4, ...,
+ * 64).  The winners are stored in
  * the context, and AUTO then follows them: a job of largest side s uses the
  * first entry whose side is at least s (the last one beyond it).  The
  * register tile is used when that entry's tile is set.  The cooperative
- * kernel (with that entry's team) is used when the batch holds no more such
- * jobs than every one of their entries' grid_max_jobs.  Choices change
+ * kernel is used when the batch holds no more such jobs than every one of
+ * their entries' grid_max_jobs.  Choices change
  * speed only: every kernel gives the same bits.  Writes up to cap entries
  * to table (may be NULL) and their number to *count.  Takes a few seconds
  * and up to about 9 GB of the HBM budget while it runs.
@@ -184,10 +186,12 @@ tci_status tci_ctx_set_rrlu_algo(tci_ctx *ctx, int32_t algo);
 typedef struct tci_rrlu_tune {
     int32_t side;            /* bucket: square matrices of this side           */
     int32_t tile;            /* 1: the register tile for these (side <= 128)   */
-    int32_t grid_team;       /* threads per workgroup of the cooperative kernel */
+    int32_t grid_team;       /* threads per workgroup of the cooperative kernel that
+                                takes this side (256 or 512 when measured; 256, 512
+                                and 1024 are accepted, the kernel goes by the shape) */
     int32_t grid_max_jobs;   /* most such jobs the cooperative kernel takes (0: none) */
     float ms_stream;         /* one matrix, streaming kernel                   */
-    float ms_grid;           /* one matrix, cooperative kernel at grid_team    */
+    float ms_grid;           /* one matrix, cooperative kernel                 */
     float ms_tile_batch;     /* 512 matrices, register tile (side <= 128)      */
     float ms_stream_batch;   /* 512 matrices, streaming kernel (side <= 128)   */
 } tci_rrlu_tune;

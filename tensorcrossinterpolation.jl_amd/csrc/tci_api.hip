@@ -82,7 +82,8 @@ struct tci_ctx {
     int pi_lds_kb;      // LDS budget for Pi matrices (KiB)
     int rrlu_algo = TCI_RRLU_AUTO;   // factorization kernel of the standalone rrLU
     std::vector<tci_rrlu_tune> tune; // measured AUTO choices (tci_ctx_autotune_rrlu), by side
-    int grid_team = 0;               // the autotuner's forced cooperative team (0: none)
+    int ncu = 0;                     // compute units
+    std::vector<uint8_t> chip_host;  // host copy of the last on-chip rrLU's tables
 };
 
 // a device-to-host copy of a finished result on the context's download
@@ -238,6 +239,7 @@ struct tci_server {
     uint32_t epoch = 0;                         // launches so far
     LdsPlan plan{};
     hipEvent_t kev = nullptr;
+    bool counted = false;                       // in g_servers
     bool running = false;
     std::vector<tci_batch *> slot;              // the request of each ring slot in flight
     std::vector<tci_batch *> pending;           // submitted and not yet returned by a poll
@@ -332,6 +334,7 @@ tci_status tci_ctx_create(tci_ctx **out, int32_t device, uint64_t hbm_budget_byt
     if (c->team != 64 && c->team != 256 && c->team != 512 && c->team != 1024) c->team = 256;
     ev = getenv("TCI_WG_PER_CU");
     c->wg_env = ev && atoi(ev) > 0 ? atoi(ev) : 0;
+    HIPCHK(hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, device));
     c->lds_cu = lds_cu;
     c->lds_blk = lds_blk;
     c->lds_wg = lds_for_team(c, c->team);
@@ -419,23 +422,26 @@ static hipStream_t pick_stream(tci_ctx *ctx)
 // ------------------------------------------------------------------- rrLU
 // The job shapes of a batched rrLU, read once, and their partition between
 // the register-tile kernel (jobs up to 128×128, when the context's
-// algorithm allows it) and the streaming one.  tile_budget: the most tile
+// algorithm allows it), the on-chip kernels and the streaming one.  tile_budget: the most tile
 // scratch (doubles) the tile jobs may take, -1 for no limit; a job past it
 // goes to the streaming kernel (the results are the same bits).
 struct LuPlan {
     std::vector<tci_lu_job> h;
-    std::vector<int32_t> tile, stream, grid;
+    std::vector<int32_t> tile, stream;
+    std::vector<ChipItem> chip, big;   // the on-chip kernels' jobs
     std::vector<int64_t> soff;
     int64_t sc_tot = 0;   // tile scratch, doubles
     int64_t mx = 0;       // largest side of any job
 };
 
-static tci_status lu_partition(tci_ctx *ctx, int64_t tile_budget, LuPlan &P, bool allow_grid = true);
+static tci_status lu_partition(tci_ctx *ctx, int64_t tile_budget, LuPlan &P, bool allow_chip = true);
 
-// the cooperative factorization takes a job of at least this many elements
-// when a batch has at most kGridMaxJobs of them (AUTO)
+// While a serving grid is resident on the device a cooperative launch waits for
+// it to leave, so then the on-chip kernels take only jobs of at least this many
+// elements, and those only when a batch has at most kGridMaxJobs of them
 constexpr int64_t kGridMinElems = (int64_t)384 * 384;
 constexpr int64_t kGridMaxJobs = 8;
+static std::atomic<int> g_servers[kMaxDevices];   // serving grids per device
 
 // reads and checks the job table (and the largest side), partitions it
 static tci_status lu_read(tci_ctx *ctx, tci_lu_job *jobs, int64_t count, LuPlan &P)
@@ -473,7 +479,7 @@ static const tci_rrlu_tune *tune_for(const tci_ctx *c, int64_t m, int64_t n)
     return &c->tune.back();
 }
 
-static tci_status lu_partition(tci_ctx *ctx, int64_t tile_budget, LuPlan &P, bool allow_grid)
+static tci_status lu_partition(tci_ctx *ctx, int64_t tile_budget, LuPlan &P, bool allow_chip)
 {
     const int64_t count = (int64_t)P.h.size();
     for (int64_t q = 0; q < count; ++q) {
@@ -499,69 +505,90 @@ static tci_status lu_partition(tci_ctx *ctx, int64_t tile_budget, LuPlan &P, boo
             P.stream.push_back((int32_t)q);
         }
     }
-    // jobs that go to the cooperative whole-chip factorization: with GRID
-    // every job that fits; with AUTO the large ones of a batch too small to
-    // fill the chip with one workgroup per job
-    if (allow_grid && (ctx->rrlu_algo == TCI_RRLU_GRID || ctx->rrlu_algo == TCI_RRLU_AUTO)) {
-        std::vector<int32_t> big, rest;
-        // tuned: the fewest jobs any of the large ones' entries allows
-        int64_t maxjobs = ctx->tune.empty() ? kGridMaxJobs : INT64_MAX;
+    // jobs that go to the on-chip kernels: with GRID every job that fits; with
+    // AUTO too, or those a tuned table sends there
+    if (allow_chip && (ctx->rrlu_algo == TCI_RRLU_GRID || ctx->rrlu_algo == TCI_RRLU_AUTO)) {
+        const bool force = ctx->rrlu_algo == TCI_RRLU_GRID;
+        const bool serving = !force && g_servers[ctx->device].load(std::memory_order_relaxed) > 0;
+        std::vector<int32_t> rest;
+        int64_t maxjobs = serving && ctx->tune.empty() ? kGridMaxJobs : INT64_MAX;
         for (int32_t q : P.stream) {
             const tci_lu_job &j = P.h[(size_t)q];
-            const bool fits = j.m >= 1 && j.n >= 1 && j.m <= kGridMaxSide && j.n <= kGridMaxSide;
             const tci_rrlu_tune *t = tune_for(ctx, j.m, j.n);
-            const bool large = t ? t->grid_max_jobs > 0 : j.m * j.n >= kGridMinElems;
-            if (fits && (ctx->rrlu_algo == TCI_RRLU_GRID || large)) {
-                big.push_back(q);
-                if (t && t->grid_max_jobs < maxjobs) maxjobs = t->grid_max_jobs;
-            } else {
-                rest.push_back(q);
-            }
+            const bool want = force || (t ? t->grid_max_jobs > 0 : !serving || j.m * j.n >= kGridMinElems);
+            ChipItem it;
+            const int k = want ? rrlu_chip_plan(j.m, j.n, ctx->ncu, &it) : 0;
+            it.job = q;
+            if (k == 1) P.chip.push_back(it);
+            else if (k == 2) P.big.push_back(it);
+            else rest.push_back(q);
+            // tuned: the fewest jobs any of these jobs' entries allows
+            if (k && t && t->grid_max_jobs < maxjobs) maxjobs = t->grid_max_jobs;
         }
-        if (ctx->rrlu_algo == TCI_RRLU_GRID || (!big.empty() && (int64_t)big.size() <= maxjobs)) {
-            P.grid = big;
+        if (force || (int64_t)(P.chip.size() + P.big.size()) <= maxjobs) {
             P.stream = rest;
+        } else {
+            P.chip.clear();
+            P.big.clear();
         }
     }
     return TCI_OK;
 }
 
-// the cooperative factorization of the grid jobs, one after the other
-static tci_status lu_run_grid(tci_ctx *ctx, tci_lu_job *jobs, const LuPlan &P)
+// One launch of an on-chip kernel over its jobs: the largest teams first, and
+// among equal teams the largest matrices, so the launch ends on small ones.
+static tci_status lu_run_chip(tci_ctx *ctx, tci_lu_job *jobs, const LuPlan &P, std::vector<ChipItem> items, int big)
 {
-    if (P.grid.empty()) return TCI_OK;
+    if (items.empty()) return TCI_OK;
     hipStream_t st = ctx->stream;
-    int64_t mx = 0;
-    for (int32_t q : P.grid) {
-        const tci_lu_job &j = P.h[(size_t)q];
-        mx = j.m * j.n > mx ? j.m * j.n : mx;
+    const auto elems = [&](const ChipItem &i) { return P.h[(size_t)i.job].m * P.h[(size_t)i.job].n; };
+    std::stable_sort(items.begin(), items.end(), [&](const ChipItem &a, const ChipItem &b) {
+        return a.S != b.S ? a.S > b.S : elems(a) > elems(b);
+    });
+    int64_t nt = 0, colcap = 0, spill = 0;
+    for (ChipItem &i : items) {
+        const tci_lu_job &j = P.h[(size_t)i.job];
+        i.first = (int32_t)nt;
+        nt += i.S;
+        colcap = j.m > colcap ? j.m : colcap;
+        if (big) spill = std::max(spill, rrlu_chip_spill(i, j.m, j.n));
     }
-    int ncu = 0;
-    HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
-    const size_t b_out = lay_align(sizeof(double) * (size_t)mx), b_cand = lay_align(rrlu_grid_cand_bytes(ncu));
+    if (nt > INT32_MAX / 2) return set_err(TCI_ERR_ARG, "too many jobs");
+    const int blocks = rrlu_chip_blocks(big, ctx->ncu, (int)nt);
+    if (blocks < items[0].S) return set_err(TCI_ERR_DEVICE, "rrlu: a team of %d workgroups does not fit", items[0].S);
+    const size_t b_items = lay_align(sizeof(ChipItem) * items.size()), b_map = lay_align(sizeof(int32_t) * (size_t)nt);
+    const size_t b_mail = lay_align((size_t)64 * (size_t)nt) + 256;
+    const size_t b_cols = lay_align(sizeof(double) * 2 * (size_t)colcap * (size_t)blocks);
+    const size_t b_spill = sizeof(double) * (size_t)spill * (size_t)blocks;
+    // (the host copy lives in the context: the next call on this stream
+    // synchronizes before it reuses it)
+    std::vector<uint8_t> &h = ctx->chip_host;
+    h.resize(b_items + b_map);
+    memcpy(h.data(), items.data(), sizeof(ChipItem) * items.size());
+    int32_t *map = (int32_t *)(h.data() + b_items);
+    for (size_t q = 0; q < items.size(); ++q)
+        for (int32_t g = 0; g < items[q].S; ++g) *map++ = (int32_t)q;
     uint8_t *d = nullptr;
-    HIPCHK(hipMallocAsync((void **)&d, b_out + b_cand + 256, st));
-    hipError_t e = hipSuccess;
-    for (int32_t q : P.grid) {
-        const tci_lu_job &j = P.h[(size_t)q];
-        // the team: the autotuner's forced one, the tuned one, or the default
-        const tci_rrlu_tune *t = tune_for(ctx, j.m, j.n);
-        const int team = ctx->grid_team ? ctx->grid_team : t ? t->grid_team : rrlu_grid_default_team();
-        const int G = rrlu_grid_blocks(ctx->device, rrlu_grid_lds(j.m, j.n), team);
-        if (G < 1 || G > ncu) {
-            e = hipErrorInvalidConfiguration;
-            break;
-        }
-        int blocks = G < (int)j.n ? G : (int)j.n;
-        int32_t *flags = (int32_t *)(d + b_out + b_cand);
-        e = hipMemsetAsync(flags, 0, sizeof(int32_t), st);
-        if (e == hipSuccess) e = launch_rrlu_grid(jobs + q, j.m, j.n, (double *)d, d + b_out, flags, blocks, team, st);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(j.A, d, sizeof(double) * (size_t)(j.m * j.n), hipMemcpyDeviceToDevice, st);
-        if (e != hipSuccess) break;
-    }
+    HIPCHK(hipMallocAsync((void **)&d, b_items + b_map + b_mail + b_cols + b_spill, st));
+    hipError_t e = hipMemcpyAsync(d, h.data(), b_items + b_map, hipMemcpyHostToDevice, st);
+    uint8_t *z = d + b_items + b_map;
+    if (e == hipSuccess) e = hipMemsetAsync(z, 0, b_mail, st);
+    ChipArgs K;
+    memset(&K, 0, sizeof K);
+    K.jobs = jobs;
+    K.items = (const ChipItem *)d;
+    K.map = (const int32_t *)(d + b_items);
+    K.ntickets = (int32_t)nt;
+    K.ticket = (uint32_t *)z;
+    K.abort_word = (uint32_t *)(z + 128);
+    K.mail = (uint64_t *)(z + 256);
+    K.cols = (double *)(z + b_mail);
+    K.colcap = colcap;
+    K.spill = (double *)(z + b_mail + b_cols);
+    K.spillcap = spill;
+    if (e == hipSuccess) e = launch_rrlu_chip(K, big, blocks, st);
     (void)hipFreeAsync(d, st);
-    if (e != hipSuccess) return set_err(TCI_ERR_DEVICE, "cooperative rrlu: %s", hipGetErrorString(e));
+    if (e != hipSuccess) return set_err(TCI_ERR_DEVICE, "on-chip rrlu: %s", hipGetErrorString(e));
     return TCI_OK;
 }
 
@@ -602,7 +629,10 @@ tci_status tci_rrlu_batched_f64(tci_ctx *ctx, tci_lu_job *jobs, int64_t count)
     std::vector<int64_t> &soff = P.soff;
     const int64_t sc_tot = P.sc_tot;
     int64_t mx;
-    ps = lu_run_grid(ctx, jobs, P);
+    ps = lu_run_chip(ctx, jobs, P, P.chip, 0);
+    if (ps != TCI_OK) return ps;
+    if (!P.chip.empty() && !P.big.empty()) HIPCHK(hipStreamSynchronize(ctx->stream));   // (chip_host is used again)
+    ps = lu_run_chip(ctx, jobs, P, P.big, 1);
     if (ps != TCI_OK) return ps;
     if (!tile.empty()) {
         uint8_t *d = nullptr;
@@ -656,7 +686,6 @@ tci_status tci_ctx_autotune_rrlu(tci_ctx *ctx, tci_rrlu_tune *table, int32_t cap
     *count = 0;
     HIPCHK(hipSetDevice(ctx->device));
     static const int kSides[] = {32, 64, 128, 256, 512, 1024, 2048, 4096};
-    static const int kTeams[] = {256, 512, 1024};
     const int algo0 = ctx->rrlu_algo;
     std::vector<tci_rrlu_tune> tuned0 = ctx->tune;
     ctx->tune.clear();
@@ -707,13 +736,12 @@ tci_status tci_ctx_autotune_rrlu(tci_ctx *ctx, tci_rrlu_tune *table, int32_t cap
         if (he == hipSuccess) he = hipMemcpy(djobs, hj.data(), sizeof(tci_lu_job) * hj.size(), hipMemcpyHostToDevice);
         if (he == hipSuccess) he = hipStreamSynchronize(ctx->stream);
         // k fresh copies of A0, then the factorization timed on the context's stream
-        auto run = [&](int algo, int team, int k, float *ms) -> bool {
+        auto run = [&](int algo, int k, float *ms) -> bool {
             for (int q = 0; q < k && he == hipSuccess; ++q)
                 he = hipMemcpyAsync((uint8_t *)W + b_mat * (size_t)q, A0, sizeof(double) * mat,
                                     hipMemcpyDeviceToDevice, ctx->stream);
             if (he != hipSuccess) return false;
             ctx->rrlu_algo = algo;
-            ctx->grid_team = team;
             he = hipEventRecord(e0, ctx->stream);
             if (he != hipSuccess) return false;
             st = tci_rrlu_batched_f64(ctx, djobs, k);
@@ -725,32 +753,25 @@ tci_status tci_ctx_autotune_rrlu(tci_ctx *ctx, tci_rrlu_tune *table, int32_t cap
         tci_rrlu_tune t;
         memset(&t, 0, sizeof t);
         t.side = s;
-        float ms = 0.0f, warm = 0.0f;
-        bool ok = run(TCI_RRLU_STREAM, 0, 1, &warm) && run(TCI_RRLU_STREAM, 0, 1, &t.ms_stream);
+        float ms = 0.0f, msk = 0.0f, warm = 0.0f;
+        bool ok = run(TCI_RRLU_STREAM, 1, &warm) && run(TCI_RRLU_STREAM, 1, &t.ms_stream);
         if (ok && s <= kTileSide) {
-            ok = run(TCI_RRLU_TILE, 0, 1, &warm) && run(TCI_RRLU_TILE, 0, 512, &t.ms_tile_batch) &&
-                 run(TCI_RRLU_STREAM, 0, 512, &t.ms_stream_batch);
+            ok = run(TCI_RRLU_TILE, 1, &warm) && run(TCI_RRLU_TILE, 512, &t.ms_tile_batch) &&
+                 run(TCI_RRLU_STREAM, 512, &t.ms_stream_batch);
             t.tile = t.ms_tile_batch < t.ms_stream_batch;
         }
-        t.ms_grid = -1.0f;
-        for (int team : kTeams) {
-            if (!ok) break;
-            ok = run(TCI_RRLU_GRID, team, 1, &warm) && run(TCI_RRLU_GRID, team, 1, &ms);
-            if (ok && (t.ms_grid < 0.0f || ms < t.ms_grid)) {
-                t.ms_grid = ms;
-                t.grid_team = team;
-            }
-        }
-        // the most jobs k for which k cooperative runs beat one streaming
+        ok = ok && run(TCI_RRLU_GRID, 1, &warm) && run(TCI_RRLU_GRID, 1, &t.ms_grid);
+        ChipItem it;
+        t.grid_team = rrlu_chip_plan(s, s, ctx->ncu, &it) == 2 ? 512 : 256;
+        // the most jobs k for which one on-chip launch of k beats one streaming
         // launch of k (a launch is never faster than its slowest job)
         for (int k = 1; ok && k <= 64; k *= 2) {
-            if ((double)k * t.ms_grid < t.ms_stream) {
-                t.grid_max_jobs = k;
-                continue;
+            ok = run(TCI_RRLU_GRID, k, &msk);
+            if (ok && msk >= t.ms_stream) {
+                ok = run(TCI_RRLU_STREAM, k, &ms);
+                if (!ok || msk >= ms) break;
             }
-            ok = run(TCI_RRLU_STREAM, 0, k, &ms);
-            if (!ok || (double)k * t.ms_grid >= ms) break;
-            t.grid_max_jobs = k;
+            if (ok) t.grid_max_jobs = k;
         }
         (void)hipFree(mem);
         mem = nullptr;
@@ -761,7 +782,6 @@ tci_status tci_ctx_autotune_rrlu(tci_ctx *ctx, tci_rrlu_tune *table, int32_t cap
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     ctx->rrlu_algo = algo0;
-    ctx->grid_team = 0;
     if (st != TCI_OK) {
         ctx->tune = tuned0;
         return st;
@@ -2257,6 +2277,7 @@ static tci_status served_query(tci_batch *b)
 
 static void server_release(tci_server *s)
 {
+    if (s->counted) g_servers[s->ctx->device].fetch_sub(1, std::memory_order_relaxed);
     if (s->kev) (void)hipEventDestroy(s->kev);
     if (s->d_g) (void)hipFree(s->d_g);
     if (s->ring) (void)hipHostFree(s->ring);
@@ -2347,6 +2368,8 @@ tci_status tci_server_start(tci_ctx *ctx, const tci_problem *shape, int32_t slot
     if (stat < 0) return fail(hipErrorInvalidValue, "serving kernel attributes");
     s->plan = make_plan(ctx, (int64_t)lds_for_team(ctx, s->team) - stat, c.mrcap, c.mrcap * c.L, sbytes, lut);
     s->slot.assign((size_t)slots, nullptr);
+    s->counted = true;
+    g_servers[ctx->device].fetch_add(1, std::memory_order_relaxed);
     *out = s;
     return TCI_OK;
 }

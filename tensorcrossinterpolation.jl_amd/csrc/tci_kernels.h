@@ -67,21 +67,36 @@ hipError_t launch_rrlu(tci_lu_job *jobs_device, int64_t count, int64_t max_side,
 constexpr int kTileSide = 128;
 hipError_t launch_rrlu_tile(tci_lu_job *jobs_device, const int32_t *idx, int64_t count, double *scratch,
                             const int64_t *soff, hipStream_t st);
-// rrlu!(A) of one matrix (each side <= kGridMaxSide) over a cooperative grid
-// of `blocks` workgroups (one per CU, rrlu_grid_blocks); the packed result
-// goes to out (m×n), the job's permutations, npivot, error and status are
-// written; cand: rrlu_grid_cand_bytes(blocks) bytes; flags: one int32, zero
-// on entry
+// rrlu!(A) of matrices held on chip by teams of workgroups
+// (tci_rrlu_chip.hip), sides up to kGridMaxSide
 constexpr int kGridMaxSide = 8192;
-size_t rrlu_grid_lds(int64_t m, int64_t n);
-// team: 256, 512 or 1024 threads (anything else: the default,
-// TCI_RRLU_GRID_TEAM or 1024); the cooperative grid size for that LDS (one
-// workgroup per CU), 0 if none fits
-int rrlu_grid_default_team();
-int rrlu_grid_blocks(int device, size_t lds, int team);
-size_t rrlu_grid_cand_bytes(int blocks);
-hipError_t launch_rrlu_grid(tci_lu_job *job, int64_t m, int64_t n, double *out, void *cand, int32_t *flags,
-                            int blocks, int team, hipStream_t st);
+struct ChipItem {
+    int32_t job;          // index into the job table
+    int32_t shape, wr;    // register shape and wave rows
+    int32_t S;            // members of the team
+    int32_t first;        // the job's first ticket (its S tickets follow each other)
+};
+struct ChipArgs {
+    tci_lu_job *jobs;
+    const ChipItem *items;
+    const int32_t *map;      // ticket → item
+    int32_t ntickets;
+    uint32_t *ticket;        // next ticket (zero on entry)
+    uint32_t *abort_word;    // zero on entry
+    uint64_t *mail;          // 8 words per ticket (zero on entry)
+    double *cols;            // 2 × colcap per workgroup (rrlu_chip_blocks of them)
+    int64_t colcap;          // rows of the tallest job
+    double *spill;           // spillcap per workgroup of the big kernel
+    int64_t spillcap;
+};
+// the team for an m×n matrix (it->shape, wr and S): 1 the two-per-CU kernel, 2
+// the big one, 0 when neither takes it
+int rrlu_chip_plan(int64_t m, int64_t n, int ncu, ChipItem *it);
+// doubles of spill a member of the big kernel needs
+int64_t rrlu_chip_spill(const ChipItem &it, int64_t m, int64_t n);
+// workgroups of a launch of ntickets tickets (0: the kernel does not fit the device)
+int rrlu_chip_blocks(int big, int ncu, int ntickets);
+hipError_t launch_rrlu_chip(const ChipArgs &K, int big, int blocks, hipStream_t st);
 // One whole TT sweep of factorizations (the host-driven sweep's steps, the
 // same operations per entry) in a single workgroup, for trains whose bonds
 // are small enough that per-bond host round trips would dominate
