@@ -197,15 +197,35 @@ static inline TCI_HD int tci_pt(const tci_point *x, int t)
     return t < x->na ? (int)x->a[t] : (int)x->b[t - x->na];
 }
 
+/* acc·2^{−L}, the quantics coordinate of the integer acc = Σ (σ_i−1) 2^{L−i} */
+static inline TCI_HD double tci_quantics_scale(int64_t acc, int L)
+{
+    double s = (double)acc;
+    while (L > 0) { int c = L > 60 ? 60 : L; s = s * (1.0 / (double)((int64_t)1 << c)); L -= c; }
+    return s;
+}
+
 /* quantics coordinate Σ (σ_i−1) 2^{−i}, exact for L <= 52 */
 static inline TCI_HD double tci_quantics_x(const tci_point *x)
 {
     int64_t acc = 0;
     for (int t = 0; t < x->L; ++t) acc = acc * 2 + (tci_pt(x, t) - 1);
-    double s = (double)acc;
-    int L = x->L;
-    while (L > 0) { int c = L > 60 ? 60 : L; s = s * (1.0 / (double)((int64_t)1 << c)); L -= c; }
-    return s;
+    return tci_quantics_scale(acc, x->L);
+}
+
+/* f of the quantics kinds at the coordinate xc */
+static inline TCI_HD double tci_quantics_value(int kind, const double *p, double xc)
+{
+    if (kind == TCI_F_QUANTICS_EXP) return p[0] * tci_exp(p[1] * xc) + p[2] * tci_exp(p[3] * xc);
+    int K = (int)p[0];
+    double f = 0.0;
+    for (int k = 0; k < K; ++k) {
+        double a = p[1 + 3 * k], c = p[2 + 3 * k], w = p[3 + 3 * k];
+        double u = xc - c;
+        f = f + a * tci_exp(-(u * u) / (2.0 * (w * w)));
+    }
+    double A = p[1 + 3 * K], F = p[2 + 3 * K];
+    return f + A * tci_cos(F * xc);
 }
 
 static inline TCI_HD double tci_functor_eval(int kind, const double *p, const int32_t *ip,
@@ -226,18 +246,7 @@ static inline TCI_HD double tci_functor_eval(int kind, const double *p, const in
         }
         return 1.0 / (1.0 + s);
     }
-    case TCI_F_QUANTICS_GAUSS_COS: {
-        double xc = tci_quantics_x(x);
-        int K = (int)p[0];
-        double f = 0.0;
-        for (int k = 0; k < K; ++k) {
-            double a = p[1 + 3 * k], c = p[2 + 3 * k], w = p[3 + 3 * k];
-            double u = xc - c;
-            f = f + a * tci_exp(-(u * u) / (2.0 * (w * w)));
-        }
-        double A = p[1 + 3 * K], F = p[2 + 3 * K];
-        return f + A * tci_cos(F * xc);
-    }
+    case TCI_F_QUANTICS_GAUSS_COS: return tci_quantics_value(TCI_F_QUANTICS_GAUSS_COS, p, tci_quantics_x(x));
     case TCI_F_GAUSS_SUM: {
         int K = (int)p[0];
         double dm1 = p[1] - 1.0;
@@ -284,10 +293,7 @@ static inline TCI_HD double tci_functor_eval(int kind, const double *p, const in
         }
         return v[0];
     }
-    case TCI_F_QUANTICS_EXP: {
-        double xc = tci_quantics_x(x);
-        return p[0] * tci_exp(p[1] * xc) + p[2] * tci_exp(p[3] * xc);
-    }
+    case TCI_F_QUANTICS_EXP: return tci_quantics_value(TCI_F_QUANTICS_EXP, p, tci_quantics_x(x));
     default:
         return 0.0 / 0.0;
     }

@@ -105,6 +105,8 @@ struct SolveDesc {
     int64_t workcap;         // doubles in work
     uint8_t *gpts;           // global-search points: nsearch × L (+ found: nsearch × L)
     double *stage;           // rrLU staging vectors in HBM: 2 × mrcap
+    double *ftab;            // per-site terms of f (Engine::build_ftab): nftab tables of L × dmax
+    int32_t nftab;           // 0: f has no such terms
     // ---- outputs (device) ----
     int64_t *ranks;
     int64_t *nglob;

@@ -30,6 +30,7 @@ struct SolveCaps {
     int32_t has_init;   // the solve starts from given pivot sets (tci_state)
     int32_t cache_log2; // memo table of f: 2^cache_log2 entries, 0 = none
     int32_t rook;       // pivotsearch = :rook (its work arrays)
+    int32_t nftab;      // tables of per-site terms of f, L × dmax doubles each (0: none)
 };
 
 // bytes of a starting-state image: the pivot sets in the set arena's own
@@ -82,6 +83,7 @@ inline void layout_solve(const SolveCaps &c, SolveDesc *D, uint8_t *in, uint8_t 
     size_t o_ckey = take(ncache * CACHE_LIMBS * 8);
     size_t o_cval = take(ncache * 8);
     size_t o_rook = take(c.rook ? 6 * mr * 4 : 0);
+    size_t o_ftab = take((size_t)c.nftab * L * (size_t)c.dmax * 8);
     *state_bytes = o;
 
     size_t r = 0;
@@ -115,6 +117,7 @@ inline void layout_solve(const SolveCaps &c, SolveDesc *D, uint8_t *in, uint8_t 
         D->cache_coef = c.cache_log2 ? (const uint64_t *)(in + o_coef) : nullptr;
     }
     D->cache_log2 = c.cache_log2;
+    D->nftab = c.nftab;
     if (base && c.cache_log2) {
         D->cache_state = (uint32_t *)(base + o_cst);
         D->cache_keys = (uint64_t *)(base + o_ckey);
@@ -136,6 +139,7 @@ inline void layout_solve(const SolveCaps &c, SolveDesc *D, uint8_t *in, uint8_t 
         D->work = (double *)(base + o_work);
         D->gpts = base + o_gpts;
         D->stage = (double *)(base + o_stage);
+        D->ftab = c.nftab ? (double *)(base + o_ftab) : nullptr;
         D->rook = c.rook ? (int32_t *)(base + o_rook) : nullptr;
     }
     if (rep) {

@@ -214,6 +214,9 @@ inline int check_state(const tci_problem &p, std::string *msg)
     return TCI_OK;
 }
 
+// most entries of a Gaussian sum's term tables (1 MiB)
+constexpr int kMaxTermTable = 1 << 17;
+
 // Returns TCI_OK or an error with *msg set.
 inline int check_problem(const tci_problem &p, SolveCaps &c, std::string *msg)
 {
@@ -276,6 +279,13 @@ inline int check_problem(const tci_problem &p, SolveCaps &c, std::string *msg)
     if (o.pivotsearch != 0 && o.pivotsearch != 1)
         return bad(TCI_ERR_ARG, "Unknown pivot search strategy. Choose from :rook, :full.");
     c.rook = o.pivotsearch;
+    // per-site terms of f (Engine::build_ftab): one table for the weighted
+    // Lorentzian, one per Gaussian of a Gaussian sum, while they stay small
+    c.nftab = 0;
+    if (p.f.kind == TCI_F_LORENTZ_WEIGHTED) c.nftab = 1;
+    if (p.f.kind == TCI_F_GAUSS_SUM && p.f.params[0] >= 1.0 &&
+        p.f.params[0] * (double)L * (double)dmax <= (double)kMaxTermTable)
+        c.nftab = (int32_t)p.f.params[0];
     return TCI_OK;
 }
 
