@@ -362,7 +362,8 @@ tci_status tci_solve_submit(tci_ctx *ctx, int32_t count, const tci_problem *prob
 
 /* The solve engine's team autotuner (no counterpart in the reference).  A
  * batch of solves runs with 256 threads per solve by default (two solves per
- * CU); larger Pi matrices can run faster with 512 or 1024, small ones with a
+ * CU), or 512 (one per CU) when it holds no more solves than there are CUs;
+ * larger Pi matrices can run faster with 512 or 1024, small ones with a
  * single wave of 64 (eight solves per CU), and the best team for one solve
  * alone is not the best for thousands.  This times `batch` copies of
  * `sample` with each team (a warm-up launch and a timed one, kernel time in

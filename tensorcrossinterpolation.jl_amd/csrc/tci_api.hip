@@ -71,6 +71,7 @@ struct tci_ctx {
     uint64_t pooled = 0;                // their bytes
     int lds_wg;         // LDS bytes (static + dynamic) a solve workgroup of the default team may use
     int team;           // threads per solve workgroup (the default team)
+    bool team_env = false;   // set by TCI_TEAM
     int lds_cu = 0, lds_blk = 0, wg_env = 0;   // LDS per CU and per workgroup; TCI_WG_PER_CU (0: unset)
     // measured solve teams (tci_ctx_autotune_solve), ascending by
     // (smallest largest-mrcap, smallest batch)
@@ -107,10 +108,14 @@ static int lds_for_team(const tci_ctx *c, int team)
 
 // the team of a batch of `count` solves whose largest Pi-row capacity is
 // max_mr: among the tuned entries at or below both, the one with the largest
-// capacity and then the largest batch; the context's default team without one
+// capacity and then the largest batch.  Without one the context's default team,
+// but 512 threads while a batch leaves CUs idle anyway: one solve per CU then
+// runs on twice the waves (one weighted Lorentzian of 40 sites, d = 16: 521 ms
+// on 256 threads, 314 on 512, 309 on 1024; one Lorentzian of 8 sites 3.27, 2.46,
+// 3.46; one quantics solve of 30 sites 21.9, 16.3, 20.9)
 static int solve_team_for(const tci_ctx *c, int max_mr, int count)
 {
-    int team = c->team;
+    int team = c->team_env ? c->team : count <= c->ncu ? 512 : c->team;
     for (const auto &e : c->solve_tune)
         if (e.mrcap <= max_mr && e.count <= count) team = e.team;
     return team;
@@ -331,6 +336,7 @@ tci_status tci_ctx_create(tci_ctx **out, int32_t device, uint64_t hbm_budget_byt
     HIPCHK(hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, device));
     const char *ev = getenv("TCI_TEAM");
     c->team = ev ? atoi(ev) : 256;
+    c->team_env = ev != nullptr;
     if (c->team != 64 && c->team != 256 && c->team != 512 && c->team != 1024) c->team = 256;
     ev = getenv("TCI_WG_PER_CU");
     c->wg_env = ev && atoi(ev) > 0 ? atoi(ev) : 0;
