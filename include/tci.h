@@ -408,6 +408,13 @@ tci_status tci_batch_indexset(tci_batch *b, int32_t i, int32_t which, int32_t si
 /* site tensor T[site] (χ_{site-1} × d × χ_site column-major). */
 tci_status tci_batch_sitetensor(tci_batch *b, int32_t i, int32_t site, int64_t *dims3,
                                 double *out, int64_t cap);
+/* Solve i's site tensors and index sets at once, in host memory of the batch,
+ * valid until tci_batch_free.  tdims: 3·L, the dims3 of every site; tensors:
+ * the site tensors back to back; counts: 4·L, counts[which·L + site-1] as
+ * tci_batch_indexset gives them; sets: the entries back to back, in the order
+ * which, site, entry. */
+tci_status tci_batch_solution(tci_batch *b, int32_t i, const int64_t **tdims, const double **tensors,
+                              const int32_t **counts, const uint8_t **sets);
 tci_status tci_batch_pivoterrors(tci_batch *b, int32_t i, double *out, int64_t cap);
 tci_status tci_batch_bonderrors(tci_batch *b, int32_t i, double *out);
 /* Evaluates solve i's tensor train where it lies in device memory (its

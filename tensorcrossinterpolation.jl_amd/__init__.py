@@ -736,6 +736,14 @@ def sample_points(localdims, n, seed=0):
 # --------------------------------------------------------------------------
 # TensorCI2 / crossinterpolate2 (tensorci2.jl)
 # --------------------------------------------------------------------------
+def _from_host(address, n, dtype):
+    """A copy of n values at a host address."""
+    out = np.empty(n, dtype)
+    if n:
+        C.memmove(out.ctypes.data, address, out.nbytes)
+    return out
+
+
 class TensorCI2:
     """Result of a device solve with the fields of TensorCI2{Float64} (tensorci2.jl:6-40).
 
@@ -765,18 +773,21 @@ class TensorCI2:
         be = np.zeros(max(L - 1, 1))
         lib.tci_batch_bonderrors(batch, i, _abi.dptr(be))
         self.bonderrors = be[:L - 1]
-        self.Iset, self.Jset = [], []
-        hI, hJ = [], []
-        for which, dst in ((0, self.Iset), (1, self.Jset), (2, hI), (3, hJ)):
-            for site in range(1, L + 1):
-                ln = site - 1 if which % 2 == 0 else L - site
-                cnt = C.c_int32()
-                buf = np.zeros(1 << 16, np.uint8)
-                lib.tci_batch_indexset(batch, i, which, site, C.byref(cnt), _abi.u8ptr(buf), len(buf))
-                if cnt.value * ln > len(buf):
-                    buf = np.zeros(cnt.value * ln, np.uint8)
-                    lib.tci_batch_indexset(batch, i, which, site, C.byref(cnt), _abi.u8ptr(buf), len(buf))
-                dst.append([list(map(int, buf[e * ln:(e + 1) * ln])) for e in range(cnt.value)])
+        pt, pT, pc, ps = C.c_void_p(), C.c_void_p(), C.c_void_p(), C.c_void_p()
+        _check(lib.tci_batch_solution(batch, i, C.byref(pt), C.byref(pT), C.byref(pc), C.byref(ps)))
+        counts = _from_host(pc.value, 4 * L, np.int32).tolist()
+        lens = [list(range(L)), list(range(L - 1, -1, -1))] * 2
+        flat = _from_host(ps.value, sum(counts[w * L + b] * lens[w][b] for w in range(4) for b in range(L)),
+                          np.uint8)
+        sets, o = [], 0
+        for w in range(4):
+            per = []
+            for b in range(L):
+                n, ln = counts[w * L + b], lens[w][b]
+                per.append(flat[o:o + n * ln].reshape(n, ln).tolist())
+                o += n * ln
+            sets.append(per)
+        self.Iset, self.Jset, hI, hJ = sets
         # Iset_history / Jset_history (tensorci2.jl:12-13): only the last
         # entry is ever read (sweep2site!, 874-877), so only it is kept
         has_hist = any(len(s) for s in hI)
@@ -784,12 +795,13 @@ class TensorCI2:
         self.Jset_history = [hJ] if has_hist else []
         self.sitetensors = []
         if self.status == 0:
-            for site in range(1, L + 1):
-                d3 = np.zeros(3, np.int64)
-                lib.tci_batch_sitetensor(batch, i, site, _abi.i64ptr(d3), None, 0)
-                out = np.zeros(max(int(np.prod(d3)), 1))
-                _check(lib.tci_batch_sitetensor(batch, i, site, _abi.i64ptr(d3), _abi.dptr(out), len(out)))
-                self.sitetensors.append(out[:int(np.prod(d3))].reshape(tuple(d3), order="F"))
+            dims = _from_host(pt.value, 3 * L, np.int64).reshape(L, 3).tolist()
+            o = 0
+            for d3 in dims:
+                n = d3[0] * d3[1] * d3[2]
+                t = _from_host(pT.value + 8 * o if n else None, n, np.float64)
+                self.sitetensors.append(t.reshape(d3, order="F"))
+                o += n
 
     def __len__(self):
         return len(self.localdims)

@@ -212,6 +212,7 @@ def lib():
                                      P(C.c_uint8), C.c_int64]
     L.tci_batch_sitetensor.argtypes = [vp, C.c_int32, C.c_int32, P(C.c_int64), P(C.c_double),
                                        C.c_int64]
+    L.tci_batch_solution.argtypes = [vp, C.c_int32, P(vp), P(vp), P(vp), P(vp)]
     L.tci_batch_pivoterrors.argtypes = [vp, C.c_int32, P(C.c_double), C.c_int64]
     L.tci_batch_bonderrors.argtypes = [vp, C.c_int32, P(C.c_double)]
     L.tci_batch_free.argtypes = [vp]
@@ -253,6 +254,7 @@ EXPORTED_SYMBOLS = [
     "tci_rrlu_f64", "tci_luci_f64", "tci_rrlu_batched_f64", "tci_pi_eval_f64", "tci_options_default",
     "tci_solve_submit", "tci_batch_query", "tci_batch_wait", "tci_batch_result",
     "tci_batch_history", "tci_batch_linkdims", "tci_batch_indexset", "tci_batch_sitetensor",
+    "tci_batch_solution",
     "tci_batch_pivoterrors", "tci_batch_bonderrors", "tci_batch_free", "tci_batch_elapsed_ms",
     "tci_batch_profile", "tci_capacity_plan", "tci_tt_evaluate_f64", "tci_batch_evaluate",
     "tci_ctx_set_rrlu_algo", "tci_ctx_autotune_rrlu", "tci_ctx_set_rrlu_tuning", "tci_ctx_autotune_solve", "tci_ctx_set_solve_tuning", "tci_rrlu_batched_noalloc_f64", "tci_batch_cachestats", "tci_batch_cachedata",

@@ -68,6 +68,7 @@ struct tci_ctx {
     uint64_t budget;
     uint64_t used;
     std::vector<PoolBuf> pool;          // cached device buffers of finished batches
+    std::vector<PoolBuf> hpool;         // cached pinned buffers of packed results
     uint64_t pooled = 0;                // their bytes
     int lds_wg;         // LDS bytes (static + dynamic) a solve workgroup of the default team may use
     int team;           // threads per solve workgroup (the default team)
@@ -191,6 +192,31 @@ static void pool_put(tci_ctx *c, void *p, size_t bytes)
     c->pooled += bytes;
 }
 
+// Pinned host buffers of packed results, kept between batches (pinning costs
+// more than the download): up to kHostPoolBytes in at most kHostPoolBufs buffers
+constexpr size_t kHostPoolBytes = (size_t)512 << 20;
+constexpr size_t kHostPoolBufs = 8;
+
+static hipError_t hpool_get(tci_ctx *c, size_t bytes, PoolBuf *out)
+{
+    for (size_t i = 0; i < c->hpool.size(); ++i)
+        if (c->hpool[i].bytes >= bytes && c->hpool[i].bytes <= 4 * bytes + (1 << 20)) {
+            *out = c->hpool[i];
+            c->hpool.erase(c->hpool.begin() + (long)i);
+            return hipSuccess;
+        }
+    out->bytes = bytes;
+    return hipHostMalloc(&out->ptr, bytes, hipHostMallocDefault);
+}
+
+static void hpool_put(tci_ctx *c, const PoolBuf &b)
+{
+    size_t tot = b.bytes;
+    for (const PoolBuf &q : c->hpool) tot += q.bytes;
+    if (tot > kHostPoolBytes || c->hpool.size() >= kHostPoolBufs) (void)hipHostFree(b.ptr);
+    else c->hpool.push_back(b);
+}
+
 // a block of a slot-level server's memory: device memory, or pinned host
 // memory with its device alias
 struct ServeChunk {
@@ -229,6 +255,18 @@ struct tci_batch {
     ServeBlock dblk{}, hblk{};         // its device block and pinned staging block
     int dcls = 0, hcls = 0;            // their size classes
     const uint8_t *h_rep_pin = nullptr;   // the report's pinned host copy
+    // the packed site tensors and index sets of the solves asked for so far
+    struct Packed {
+        const double *T = nullptr;
+        const uint8_t *sets = nullptr;
+        std::vector<int64_t> tdims;    // 3·L
+        std::vector<int32_t> counts;   // 4·L
+        std::vector<int64_t> off;      // 5·L: byte offsets of a site's tensor (from T) and sets (from sets)
+    };
+    std::vector<Packed> packed;
+    std::vector<PoolBuf> packs;            // their pinned buffers
+    std::vector<std::vector<uint8_t>> hostpacks;   // of served requests: ordinary memory
+    int npacked = 0;
 };
 
 // A slot-level server: the persistent serving grid and its queue.
@@ -360,6 +398,7 @@ tci_status tci_ctx_destroy(tci_ctx *ctx)
         (void)hipStreamDestroy(s);
     }
     for (PoolBuf &b : ctx->pool) (void)hipFree(b.ptr);
+    for (PoolBuf &b : ctx->hpool) (void)hipHostFree(b.ptr);
     (void)hipStreamDestroy(ctx->dl);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -1490,6 +1529,10 @@ static void batch_release(tci_batch *b)
     }
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
+    for (const PoolBuf &q : b->packs) {
+        if (b->ctx) hpool_put(b->ctx, q);
+        else (void)hipHostFree(q.ptr);
+    }
     delete b;
 }
 
@@ -1750,6 +1793,7 @@ static bool report_view(tci_batch *b, int32_t i, SolveDesc &R)
     R.pivoterrors = (double *)h(R.pivoterrors);
     R.bonderrors = (double *)h(R.bonderrors);
     R.setn = (int32_t *)h(R.setn);
+    R.Tdims = (int64_t *)h(R.Tdims);
     return true;
 }
 
@@ -1787,26 +1831,159 @@ tci_status tci_batch_linkdims(tci_batch *b, int32_t i, int64_t *linkdims)
     return TCI_OK;
 }
 
+// The four index sets a solve is asked for: the kind of `which` (0 Iset, 1 Jset,
+// 2 and 3 their last history entries, in the slot the solve wrote last)
+static int set_kind(const SolveDesc &R, int which)
+{
+    const bool jside = which & 1;
+    if (which < 2) return jside ? SET_J : SET_I;
+    return R.ints[INT_HIST] == 2 ? (jside ? SET_HB_J : SET_HB_I) : (jside ? SET_HA_J : SET_HA_I);
+}
+static int set_count(const SolveDesc &R, int which, int b)
+{
+    return which >= 2 && R.ints[INT_HIST] == 0 ? 0 : R.setn[set_kind(R, which) * R.L + b];
+}
+static int set_len(const SolveDesc &R, int which, int b) { return (which & 1) ? R.L - 1 - b : b; }
+
+// The shape of solve i's packed results, from its report; returns their bytes
+// (tensors, then sets).
+static size_t pack_shape(const SolveDesc &R, tci_batch::Packed &P, size_t *tensor_bytes)
+{
+    const int L = R.L;
+    P.tdims.assign(R.Tdims, R.Tdims + 3 * L);
+    P.counts.resize((size_t)4 * L);
+    P.off.resize((size_t)5 * L);
+    int64_t o = 0;
+    for (int b = 0; b < L; ++b) {
+        P.off[(size_t)5 * b] = o;
+        o += 8 * P.tdims[(size_t)3 * b] * P.tdims[(size_t)3 * b + 1] * P.tdims[(size_t)3 * b + 2];
+    }
+    *tensor_bytes = (size_t)o;
+    int64_t s = 0;
+    for (int w = 0; w < 4; ++w)
+        for (int b = 0; b < L; ++b) {
+            P.counts[(size_t)w * L + b] = set_count(R, w, b);
+            P.off[(size_t)5 * b + 1 + w] = s;
+            s += (int64_t)P.counts[(size_t)w * L + b] * set_len(R, w, b);
+        }
+    return (size_t)o + (((size_t)s + 15) & ~(size_t)15);
+}
+
+constexpr size_t kPackGroupBytes = (size_t)1 << 30;
+
+// Solve i's site tensors and index sets in host memory.  The first solve asked
+// for is packed alone; when another one follows, all the others come with it (a
+// download per tensor and set costs 25 us each, and a batch of 384 solves has
+// 15 000 of them: 640 ms against 3 for the solves themselves), up to 1 GiB at a
+// time.  A served request is read directly: its pack kernel could have to wait
+// for the resident grid.
+static tci_status ensure_packed(tci_batch *b, int32_t i)
+{
+    SolveDesc R;
+    if (!report_view(b, i, R)) return set_err(TCI_ERR_ARG, "bad batch/index");
+    if (b->packed.empty()) b->packed.resize((size_t)b->count);
+    if (!b->packed[(size_t)i].counts.empty()) return TCI_OK;
+    tci_ctx *ctx = b->ctx;
+    HIPCHK(hipSetDevice(ctx->device));
+    size_t tb = 0;
+    if (b->served) {
+        tci_batch::Packed P;
+        const size_t bytes = pack_shape(R, P, &tb);
+        std::vector<uint8_t> h(bytes ? bytes : 1);
+        std::vector<uint8_t> raw;
+        for (int s = 0; s < R.L; ++s) {
+            const int64_t n = P.tdims[(size_t)3 * s] * P.tdims[(size_t)3 * s + 1] * P.tdims[(size_t)3 * s + 2];
+            if (n > 0) HIPCHK(ctx_download(ctx, h.data() + P.off[(size_t)5 * s], R.T + R.tstride * s, sizeof(double) * n));
+            for (int w = 0; w < 4; ++w) {
+                const int cnt = P.counts[(size_t)w * R.L + s], len = set_len(R, w, s);
+                if (cnt == 0 || len == 0) continue;
+                raw.resize((size_t)cnt * R.L);
+                const uint8_t *src = R.sets + ((int64_t)(set_kind(R, w) * R.L + s) * R.setcap) * R.L;
+                HIPCHK(ctx_download(ctx, raw.data(), src, raw.size()));
+                uint8_t *dst = h.data() + tb + P.off[(size_t)5 * s + 1 + w];
+                for (int e = 0; e < cnt; ++e) memcpy(dst + (size_t)e * len, raw.data() + (size_t)e * R.L, (size_t)len);
+            }
+        }
+        b->hostpacks.push_back(std::move(h));
+        P.T = (const double *)b->hostpacks.back().data();
+        P.sets = b->hostpacks.back().data() + tb;
+        b->packed[(size_t)i] = std::move(P);
+        return TCI_OK;
+    }
+    // the group to pack: i, and from the second solve on every other one left
+    std::vector<int32_t> solve(1, i);
+    std::vector<tci_batch::Packed> P(1);
+    std::vector<size_t> start(1, 0), tbs(1, 0);
+    size_t total = pack_shape(R, P[0], &tbs[0]);
+    int L0 = R.L;
+    if (b->npacked > 0)
+        for (int32_t q = 0; q < b->count; ++q) {
+            if (q == i || !b->packed[(size_t)q].counts.empty()) continue;
+            SolveDesc Q;
+            if (!report_view(b, q, Q)) continue;
+            tci_batch::Packed p;
+            const size_t bytes = pack_shape(Q, p, &tb);
+            if (total + bytes > kPackGroupBytes) break;
+            solve.push_back(q);
+            P.push_back(std::move(p));
+            start.push_back(total);
+            tbs.push_back(tb);
+            total += bytes;
+            L0 = Q.L > L0 ? Q.L : L0;
+        }
+    const size_t n = solve.size();
+    if (n * (size_t)L0 > (size_t)INT32_MAX) return set_err(TCI_ERR_ARG, "too many solves");
+    std::vector<int64_t> at(5 * n * (size_t)L0, 0);
+    for (size_t q = 0; q < n; ++q)
+        for (size_t s = 0; 5 * s < P[q].off.size(); ++s)
+            for (size_t w = 0; w < 5; ++w)
+                at[5 * (q * (size_t)L0 + s) + w] =
+                    (int64_t)start[q] + (w ? (int64_t)tbs[q] : 0) + P[q].off[5 * s + w];
+    const size_t b_idx = lay_align(sizeof(int32_t) * n), b_at = lay_align(sizeof(int64_t) * at.size());
+    void *dev = nullptr;
+    size_t got = 0;
+    PoolBuf host{nullptr, 0};
+    hipError_t e = pool_get(ctx, b_idx + b_at + total + 16, &dev, &got);
+    if (e != hipSuccess) return set_err(TCI_ERR_OOM, "packed results: %s", hipGetErrorString(e));
+    uint8_t *d = (uint8_t *)dev;
+    e = hpool_get(ctx, total + 16, &host);
+    if (e == hipSuccess) e = hipMemcpyAsync(d, solve.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, ctx->dl);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(d + b_idx, at.data(), sizeof(int64_t) * at.size(), hipMemcpyHostToDevice, ctx->dl);
+    if (e == hipSuccess)
+        e = launch_pack(b->d_desc, (const int32_t *)d, (int)n, L0, (const int64_t *)(d + b_idx), d + b_idx + b_at, ctx->dl);
+    if (e == hipSuccess && total)
+        e = hipMemcpyAsync(host.ptr, d + b_idx + b_at, total, hipMemcpyDeviceToHost, ctx->dl);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->dl);
+    pool_put(ctx, dev, got);
+    if (e != hipSuccess) {
+        if (host.ptr) hpool_put(ctx, host);
+        return set_err(TCI_ERR_DEVICE, "packed results: %s", hipGetErrorString(e));
+    }
+    b->packs.push_back(host);
+    for (size_t q = 0; q < n; ++q) {
+        P[q].T = (const double *)((const uint8_t *)host.ptr + start[q]);
+        P[q].sets = (const uint8_t *)host.ptr + start[q] + tbs[q];
+        b->packed[(size_t)solve[q]] = std::move(P[q]);
+    }
+    b->npacked += (int)n;
+    return TCI_OK;
+}
+
 tci_status tci_batch_indexset(tci_batch *b, int32_t i, int32_t which, int32_t site, int32_t *count,
                               uint8_t *out, int64_t cap_bytes)
 {
     SolveDesc R;
     if (!count || !report_view(b, i, R) || site < 1 || site > R.L || which < 0 || which > 3)
         return set_err(TCI_ERR_ARG, "bad arguments");
-    const int L = R.L, b0 = site - 1, jside = which & 1;
-    // which 2/3: the last history entry, in the slot the solve wrote last
-    const int hist = R.ints[INT_HIST];
-    const int kind = which < 2 ? (jside ? SET_J : SET_I)
-                               : (hist == 2 ? (jside ? SET_HB_J : SET_HB_I) : (jside ? SET_HA_J : SET_HA_I));
-    const int len = jside ? L - 1 - b0 : b0;
-    const int n = (which >= 2 && hist == 0) ? 0 : R.setn[kind * L + b0];
+    const int b0 = site - 1, len = set_len(R, which, b0), n = set_count(R, which, b0);
     *count = n;
     if ((int64_t)n * len > cap_bytes || (!out && n * len > 0)) return set_err(TCI_ERR_ARG, "output buffer too small");
     if (n == 0 || len == 0) return TCI_OK;
-    std::vector<uint8_t> raw((size_t)n * L);
-    const uint8_t *src = R.sets + ((int64_t)(kind * L + b0) * R.setcap) * L;
-    HIPCHK(ctx_download(b->ctx, raw.data(), src, raw.size()));
-    for (int e = 0; e < n; ++e) memcpy(out + (size_t)e * len, raw.data() + (size_t)e * L, (size_t)len);
+    const tci_status s = ensure_packed(b, i);
+    if (s != TCI_OK) return s;
+    const tci_batch::Packed &P = b->packed[(size_t)i];
+    memcpy(out, P.sets + P.off[(size_t)5 * b0 + 1 + which], (size_t)n * len);
     return TCI_OK;
 }
 
@@ -1814,10 +1991,29 @@ tci_status tci_batch_sitetensor(tci_batch *b, int32_t i, int32_t site, int64_t *
 {
     SolveDesc R;
     if (!dims3 || !report_view(b, i, R) || site < 1 || site > R.L) return set_err(TCI_ERR_ARG, "bad arguments");
-    HIPCHK(ctx_download(b->ctx, dims3, R.Tdims + 3 * (site - 1), sizeof(int64_t) * 3));
+    for (int k = 0; k < 3; ++k) dims3[k] = R.Tdims[3 * (site - 1) + k];
     const int64_t n = dims3[0] * dims3[1] * dims3[2];
     if (n > cap || (!out && n > 0)) return set_err(TCI_ERR_ARG, "output buffer too small");
-    if (n > 0) HIPCHK(ctx_download(b->ctx, out, R.T + R.tstride * (site - 1), sizeof(double) * n));
+    if (n == 0) return TCI_OK;
+    const tci_status s = ensure_packed(b, i);
+    if (s != TCI_OK) return s;
+    const tci_batch::Packed &P = b->packed[(size_t)i];
+    memcpy(out, (const uint8_t *)P.T + P.off[(size_t)5 * (site - 1)], sizeof(double) * (size_t)n);
+    return TCI_OK;
+}
+
+tci_status tci_batch_solution(tci_batch *b, int32_t i, const int64_t **tdims, const double **tensors,
+                              const int32_t **counts, const uint8_t **sets)
+{
+    if (!tdims || !tensors || !counts || !sets) return set_err(TCI_ERR_ARG, "bad arguments");
+    if (!b || i < 0 || i >= b->count) return set_err(TCI_ERR_ARG, "bad batch/index");
+    const tci_status s = ensure_packed(b, i);
+    if (s != TCI_OK) return s;
+    const tci_batch::Packed &P = b->packed[(size_t)i];
+    *tdims = P.tdims.data();
+    *tensors = P.T;
+    *counts = P.counts.data();
+    *sets = P.sets;
     return TCI_OK;
 }
 
@@ -2110,7 +2306,7 @@ tci_status tci_batch_evaluate(tci_batch *b, int32_t i, int64_t npts, const uint8
     std::vector<int32_t> ld((size_t)L);
     std::vector<int64_t> dims3((size_t)(3 * L)), coff((size_t)L);
     HIPCHK(ctx_download(ctx, ld.data(), R.localdims, sizeof(int32_t) * (size_t)L));
-    HIPCHK(ctx_download(ctx, dims3.data(), R.Tdims, sizeof(int64_t) * dims3.size()));
+    HIPCHK(ctx_download(ctx, dims3.data(), b->desc[(size_t)i].Tdims, sizeof(int64_t) * dims3.size()));
     if (!points_in_range(L, ld.data(), npts, pts)) return set_err(TCI_ERR_ARG, "point index out of range");
     int64_t chimax = 1;
     for (int s = 0; s < L; ++s) {
@@ -2124,7 +2320,7 @@ tci_status tci_batch_evaluate(tci_batch *b, int32_t i, int64_t npts, const uint8
     hipError_t e = hipMemcpyAsync(d_off, coff.data(), sizeof(int64_t) * coff.size(), hipMemcpyHostToDevice, st);
     tci_status s = TCI_OK;
     if (e != hipSuccess) s = set_err(TCI_ERR_DEVICE, "offsets upload: %s", hipGetErrorString(e));
-    else s = tt_eval_device(ctx, st, L, R.Tdims, d_off, R.T, (int)chimax, npts, pts, R.fkind, R.params,
+    else s = tt_eval_device(ctx, st, L, b->desc[(size_t)i].Tdims, d_off, R.T, (int)chimax, npts, pts, R.fkind, R.params,
                             R.iparams, tt_out, f_out, maxerr, maxabsf);
     (void)hipFreeAsync(d_off, st);
     (void)hipStreamSynchronize(st);

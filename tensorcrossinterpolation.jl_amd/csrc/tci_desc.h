@@ -100,7 +100,7 @@ struct SolveDesc {
     double *pivval;          // mrcap
     double *T;               // L site-tensor slots of tstride doubles
     int64_t tstride;
-    int64_t *Tdims;          // 3L
+    int64_t *Tdims;          // 3L (in the report)
     double *work;            // global-search scratch
     int64_t workcap;         // doubles in work
     uint8_t *gpts;           // global-search points: nsearch × L (+ found: nsearch × L)

@@ -62,6 +62,12 @@ hipError_t launch_serve(const ServeSlot *ring, ServeDev *g, const ServeCtl *ctl,
 // order (device, count entries, or null): the job index each workgroup takes
 hipError_t launch_rrlu(tci_lu_job *jobs_device, int64_t count, int64_t max_side, double *gstage,
                        int64_t gstage_stride, const int32_t *order, hipStream_t st);
+// The site tensors and index sets of finished solves, packed for one download:
+// block (q, site) copies solve[q]'s site tensor and its four index sets (Iset,
+// Jset and their last history entries, entries back to back) to out + the five
+// byte offsets at[5·(q·L0 + site) ...]; L0: the largest L of the solves.
+hipError_t launch_pack(const SolveDesc *descs, const int32_t *solve, int count, int L0, const int64_t *at,
+                       uint8_t *out, hipStream_t st);
 // the register-tile rrLU of the jobs idx[0..count) (each m, n <= 128);
 // scratch + soff[q]: m·mr + mr·n doubles for job idx[q] (mr = min(m, n, maxrank))
 constexpr int kTileSide = 128;

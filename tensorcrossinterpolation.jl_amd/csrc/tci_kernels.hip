@@ -239,6 +239,46 @@ hipError_t launch_serve(const ServeSlot *ring, ServeDev *g, const ServeCtl *ctl,
     return hipGetLastError();
 }
 
+// ------------------------------------------------------- packed results
+// at: 5 byte offsets per (solve, site): the tensor, then Iset, Jset and their
+// last history entries
+__global__ __launch_bounds__(256) void tci_pack_kernel(const SolveDesc *__restrict__ descs,
+                                                       const int32_t *__restrict__ solve, int L0,
+                                                       const int64_t *__restrict__ at, uint8_t *__restrict__ out)
+{
+    const int q = blockIdx.x / L0, b = blockIdx.x - q * L0;
+    const SolveDesc &D = descs[solve[q]];
+    const int L = D.L;
+    if (b >= L) return;
+    const int64_t *o = at + 5 * ((int64_t)q * L0 + b);
+    const int64_t n = D.Tdims[3 * b] * D.Tdims[3 * b + 1] * D.Tdims[3 * b + 2];
+    const double *T = D.T + D.tstride * b;
+    double *dst = (double *)(out + o[0]);
+    for (int64_t e = threadIdx.x; e < n; e += blockDim.x) dst[e] = T[e];
+    const int hist = D.ints[INT_HIST];
+    for (int w = 0; w < 4; ++w) {
+        const bool jside = w & 1;
+        if (w >= 2 && hist == 0) break;
+        const int kind = w < 2 ? (jside ? SET_J : SET_I)
+                               : (hist == 2 ? (jside ? SET_HB_J : SET_HB_I) : (jside ? SET_HA_J : SET_HA_I));
+        const int len = jside ? L - 1 - b : b, cnt = D.setn[kind * L + b];
+        const uint8_t *src = D.sets + ((int64_t)(kind * L + b) * D.setcap) * L;
+        uint8_t *d = out + o[1 + w];
+        for (int e = threadIdx.x; e < cnt * len; e += blockDim.x) {
+            const int r = e / len, t = e - r * len;
+            d[e] = src[(int64_t)r * L + t];
+        }
+    }
+}
+
+hipError_t launch_pack(const SolveDesc *descs, const int32_t *solve, int count, int L0, const int64_t *at,
+                       uint8_t *out, hipStream_t st)
+{
+    if (count < 1) return hipSuccess;
+    hipLaunchKernelGGL(tci_pack_kernel, dim3((unsigned)(count * L0)), dim3(256), 0, st, descs, solve, L0, at, out);
+    return hipGetLastError();
+}
+
 // ------------------------------------------------------------------ rrLU
 // order: the job each workgroup takes (largest first, so the long
 // factorizations start early and the launch ends evenly), or null

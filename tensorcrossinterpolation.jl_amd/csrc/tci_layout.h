@@ -74,7 +74,6 @@ inline void layout_solve(const SolveCaps &c, SolveDesc *D, uint8_t *in, uint8_t 
     size_t o_ipiv = take(2 * sc * 4);
     size_t o_pv = take(mr * 8);
     size_t o_T = take(L * tstride * 8);
-    size_t o_Td = take(3 * L * 8);
     size_t o_work = take(ncand * (1 + 2 * sc) * 8);
     size_t o_gpts = take((2 * (size_t)c.nsearch + ncand) * L);
     size_t o_stage = take(2 * mr * 8);
@@ -96,6 +95,7 @@ inline void layout_solve(const SolveCaps &c, SolveDesc *D, uint8_t *in, uint8_t 
     size_t r_pe = rtake((sc + 2) * 8);
     size_t r_be = rtake(L * 8);
     size_t r_setn = rtake((size_t)NSETKIND * L * 4);
+    size_t r_Td = rtake(3 * L * 8);
     *report_bytes = lay_align(r);
 
     if (!D) return;
@@ -135,7 +135,6 @@ inline void layout_solve(const SolveCaps &c, SolveDesc *D, uint8_t *in, uint8_t 
         D->ipiv = (int32_t *)(base + o_ipiv);
         D->pivval = (double *)(base + o_pv);
         D->T = (double *)(base + o_T);
-        D->Tdims = (int64_t *)(base + o_Td);
         D->work = (double *)(base + o_work);
         D->gpts = base + o_gpts;
         D->stage = (double *)(base + o_stage);
@@ -151,6 +150,7 @@ inline void layout_solve(const SolveCaps &c, SolveDesc *D, uint8_t *in, uint8_t 
         D->pivoterrors = (double *)(rep + r_pe);
         D->bonderrors = (double *)(rep + r_be);
         D->setn = (int32_t *)(rep + r_setn);
+        D->Tdims = (int64_t *)(rep + r_Td);
     }
 }
 
