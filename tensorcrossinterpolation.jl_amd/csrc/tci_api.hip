@@ -2127,27 +2127,81 @@ static bool points_in_range(int L, const int32_t *localdims, int64_t npts, const
 
 // device part shared by the two TT evaluation entry points: points upload,
 // launch, results back; dims3/coff/cores/params are device pointers
-static tci_status tt_eval_device(tci_ctx *ctx, hipStream_t st, int L, const int64_t *d_dims3,
+// The two routes of a TT evaluation: one launch whose workgroups take a few
+// points each through every site, and, for many points, one launch per site
+// over points grouped by local index (tci_tt_site_kernel).  The second pays for
+// its launches and its sorting from about 10^6 products on, where the bonds are
+// wide enough to hold a wave's columns.  Whole calls, first / second, ms: 20
+// sites, d = 10, bond 16: 300 points 0.86 / 0.36, 100 000 points 1.67 / 1.22; bond
+// 96: 300 points 5.7 / 3.5, 100 000 points 55.9 / 6.2; bond 3: 100 000 points 0.71
+// / 0.98; 5 sites, bond 7, 5000 points 0.15 / 0.22.
+static bool tt_grouped(int64_t npts, int L, const std::vector<int64_t> &dims3, int64_t chimax)
+{
+    int64_t macs = 0;
+    for (int b = 0; b < L; ++b) macs += dims3[(size_t)(3 * b)] * dims3[(size_t)(3 * b + 2)];
+    return chimax <= kTtSiteMax && macs >= 40 * (int64_t)L && npts * macs >= 1000000;
+}
+
+constexpr size_t kTtVecBytes = (size_t)512 << 20;   // running vectors of one chunk of points
+
+static tci_status tt_eval_device(tci_ctx *ctx, hipStream_t st, int L, const std::vector<int64_t> &dims3,
+                                 const std::vector<int64_t> &coff, const int64_t *d_dims3,
                                  const int64_t *d_coff, const double *d_cores, int chimax, int64_t npts,
                                  const uint8_t *pts, int fkind, const double *d_params,
                                  const int32_t *d_iparams, double *tt_out, double *f_out, double *maxerr,
                                  double *maxabsf)
 {
-    const int np = tt_eval_points_per_block(chimax);
+    const bool grouped = tt_grouped(npts, L, dims3, chimax);
+    int64_t chunk = npts, dmax = 1;
+    if (grouped) {
+        chunk = std::max((int64_t)64, (int64_t)(kTtVecBytes / (16 * (size_t)chimax)) & ~(int64_t)255);
+        chunk = std::min(npts, chunk);
+        for (int b = 0; b < L; ++b) dmax = std::max(dmax, dims3[(size_t)(3 * b + 1)]);
+    }
+    const int np = grouped ? 256 : tt_eval_points_per_block(chimax);
     const int64_t blocks = (npts + np - 1) / np;
+    const int64_t maxtiles = chunk / 64 + dmax + 1;
+    if (grouped && maxtiles > INT32_MAX) return set_err(TCI_ERR_ARG, "too many points");
     size_t need = 0;
     auto a = [&](size_t bytes) { size_t at = need; need = lay_align(need + (bytes ? bytes : 1)); return at; };
     const size_t o_pts = a((size_t)(npts * L));
     const size_t o_tt = a(sizeof(double) * (size_t)npts);
     const size_t o_f = a(sizeof(double) * (size_t)npts);
     const size_t o_bm = a(sizeof(double) * (size_t)(2 * blocks));
+    const size_t o_bins = a(grouped ? sizeof(int32_t) * 256 * (size_t)L : 0);
+    const size_t o_nt = a(grouped ? sizeof(int32_t) * (size_t)L : 0);
+    const size_t o_tiles = a(grouped ? sizeof(TtTile) * (size_t)maxtiles * (size_t)L : 0);
+    const size_t o_ord = a(grouped ? sizeof(int32_t) * (size_t)chunk * (size_t)L : 0);
+    const size_t o_v = a(grouped ? sizeof(double) * (size_t)chunk * (size_t)chimax : 0);
+    const size_t o_w = a(grouped ? sizeof(double) * (size_t)chunk * (size_t)chimax : 0);
     uint8_t *d = nullptr;
     HIPCHK(hipMallocAsync((void **)&d, need, st));
     hipError_t e = hipMemcpyAsync(d + o_pts, pts, (size_t)(npts * L), hipMemcpyHostToDevice, st);
-    if (e == hipSuccess)
+    if (!grouped && e == hipSuccess)
         e = launch_tt_eval(L, d_dims3, d_coff, d_cores, d + o_pts, npts, chimax, fkind, d_params, d_iparams,
                            (double *)(d + o_tt), fkind ? (double *)(d + o_f) : nullptr,
                            (double *)(d + o_bm), st);
+    for (int64_t q0 = 0; grouped && q0 < npts && e == hipSuccess; q0 += chunk) {
+        const int64_t n = std::min(chunk, npts - q0);
+        const uint8_t *dp = d + o_pts + q0 * L;
+        const TtTile *tiles = (const TtTile *)(d + o_tiles);
+        const int32_t *order = (const int32_t *)(d + o_ord), *nt = (const int32_t *)(d + o_nt);
+        e = hipMemsetAsync(d + o_bins, 0, sizeof(int32_t) * 256 * (size_t)L, st);
+        if (e == hipSuccess)
+            e = launch_tt_group(dp, n, L, (int32_t *)(d + o_bins), (TtTile *)(d + o_tiles), (int32_t *)(d + o_nt),
+                                (int)maxtiles, (int32_t *)(d + o_ord), st);
+        double *V = (double *)(d + o_v), *W = (double *)(d + o_w);
+        for (int b = 0; b < L && e == hipSuccess; ++b) {
+            const int64_t *dd = dims3.data() + 3 * b;
+            e = launch_tt_site(d_cores + coff[(size_t)b], (int)dd[0], (int)dd[1], (int)dd[2],
+                               tiles + (int64_t)b * maxtiles, nt + b, (int)(n / 64 + dd[1] + 1), order + (int64_t)b * n,
+                               b ? V : nullptr, W, chimax, st);
+            std::swap(V, W);
+        }
+        if (e == hipSuccess)
+            e = launch_tt_finish(V, chimax, dp, n, L, fkind, d_params, d_iparams, (double *)(d + o_tt) + q0,
+                                 fkind ? (double *)(d + o_f) + q0 : nullptr, (double *)(d + o_bm) + 2 * (q0 / 256), st);
+    }
     std::vector<double> bm;
     if (e == hipSuccess && tt_out)
         e = hipMemcpyAsync(tt_out, d + o_tt, sizeof(double) * (size_t)npts, hipMemcpyDeviceToHost, st);
@@ -2208,7 +2262,7 @@ tci_status tci_tt_evaluate_f64(tci_ctx *ctx, int32_t L, const int64_t *linkdims,
     if (e == hipSuccess) e = hipMemcpyAsync(d + o_o, coff.data(), sizeof(int64_t) * coff.size(), hipMemcpyHostToDevice, st);
     tci_status s = TCI_OK;
     if (e != hipSuccess) s = set_err(TCI_ERR_DEVICE, "TT upload: %s", hipGetErrorString(e));
-    else s = tt_eval_device(ctx, st, L, (const int64_t *)(d + o_d), (const int64_t *)(d + o_o),
+    else s = tt_eval_device(ctx, st, L, dims3, coff, (const int64_t *)(d + o_d), (const int64_t *)(d + o_o),
                             (const double *)(d + o_c), (int)chimax, npts, pts, 0, nullptr, nullptr, out,
                             nullptr, nullptr, nullptr);
     (void)hipFreeAsync(d, st);
@@ -2320,7 +2374,7 @@ tci_status tci_batch_evaluate(tci_batch *b, int32_t i, int64_t npts, const uint8
     hipError_t e = hipMemcpyAsync(d_off, coff.data(), sizeof(int64_t) * coff.size(), hipMemcpyHostToDevice, st);
     tci_status s = TCI_OK;
     if (e != hipSuccess) s = set_err(TCI_ERR_DEVICE, "offsets upload: %s", hipGetErrorString(e));
-    else s = tt_eval_device(ctx, st, L, b->desc[(size_t)i].Tdims, d_off, R.T, (int)chimax, npts, pts, R.fkind, R.params,
+    else s = tt_eval_device(ctx, st, L, dims3, coff, b->desc[(size_t)i].Tdims, d_off, R.T, (int)chimax, npts, pts, R.fkind, R.params,
                             R.iparams, tt_out, f_out, maxerr, maxabsf);
     (void)hipFreeAsync(d_off, st);
     (void)hipStreamSynchronize(st);

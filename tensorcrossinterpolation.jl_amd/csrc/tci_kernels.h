@@ -145,6 +145,23 @@ hipError_t launch_tt_eval(int L, const int64_t *dims3, const int64_t *coff, cons
                           const uint8_t *pts, int64_t npts, int chimax, int fkind, const double *params,
                           const int32_t *iparams, double *out_tt, double *out_f, double *blockmax,
                           hipStream_t st);
+// TT evaluation of many points, site by site over points grouped by local index:
+// bins (256 per site, zero on entry), tiles and ntiles (maxtiles >= npts/64 + the
+// largest local dimension, per site) and order (npts per site) are filled by
+// launch_tt_group; launch_tt_site forms one site's vectors W from V (stride
+// doubles per point; V null at the first site) for d0 <= kTtSiteMax;
+// launch_tt_finish reads V's first entries out (two block maxima per 256 points)
+struct TtTile {
+    int32_t s, first, n;
+};
+constexpr int kTtSiteMax = 256;
+hipError_t launch_tt_group(const uint8_t *pts, int64_t npts, int L, int32_t *bins, TtTile *tiles, int32_t *ntiles,
+                           int maxtiles, int32_t *order, hipStream_t st);
+hipError_t launch_tt_site(const double *T, int d0, int d, int d2, const TtTile *tiles, const int32_t *ntiles,
+                          int maxtiles, const int32_t *order, const double *V, double *W, int stride, hipStream_t st);
+hipError_t launch_tt_finish(const double *V, int stride, const uint8_t *pts, int64_t npts, int L, int fkind,
+                            const double *params, const int32_t *iparams, double *out_tt, double *out_f,
+                            double *blockmax, hipStream_t st);
 // _floatingzone from each of npts points (in/out, npts×L digits), one
 // workgroup per point; work: wstride doubles per workgroup, digits: dmax·L
 // bytes per workgroup; roff: L+1 offsets of the right environments

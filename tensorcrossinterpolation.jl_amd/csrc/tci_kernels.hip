@@ -802,6 +802,218 @@ __global__ __launch_bounds__(256) void tci_tt_eval_kernel(
     }
 }
 
+// ---- many points at once.  Per site the points are grouped by their local
+// index s, so that 64 of them share the slice T_b[:, s, :]: a lane carries one
+// point, the slice's entries come through scalar loads, and every LDS read of
+// the running vector feeds J products.  tci_tt_eval_kernel above loads one core
+// entry per product, each lane from another column: 53 ms for 100 000 points of
+// 20 sites, d = 10, bond dimension 96; these 3.3 ms together (0.85 ms is the rate
+// of unfused FP64 multiplies and adds).
+constexpr int kTtBins = 256;    // local indices are 1..255
+
+__global__ __launch_bounds__(256) void tci_tt_count_kernel(const uint8_t *__restrict__ pts, int64_t npts, int L,
+                                                           int32_t *__restrict__ bins)
+{
+    __shared__ int32_t h[kTtBins];
+    const int b = blockIdx.y;
+    h[threadIdx.x] = 0;
+    __syncthreads();
+    for (int u = 0; u < 4; ++u) {
+        const int64_t q = (int64_t)blockIdx.x * 1024 + u * 256 + threadIdx.x;
+        if (q < npts) atomicAdd(&h[pts[q * L + b]], 1);
+    }
+    __syncthreads();
+    if (h[threadIdx.x]) atomicAdd(&bins[b * kTtBins + threadIdx.x], h[threadIdx.x]);
+}
+
+// per site: bins[s] becomes the first place of s's points, and the tiles of at
+// most 64 points of one s are listed
+__global__ __launch_bounds__(256) void tci_tt_tiles_kernel(int32_t *__restrict__ bins, TtTile *__restrict__ tiles,
+                                                           int32_t *__restrict__ ntiles, int maxtiles)
+{
+    __shared__ int32_t place[kTtBins], tile[kTtBins];
+    const int b = blockIdx.x, s = threadIdx.x;
+    const int n = bins[b * kTtBins + s], t = (n + 63) / 64;
+    place[s] = n;
+    tile[s] = t;
+    __syncthreads();
+    for (int off = 1; off < kTtBins; off *= 2) {
+        const int x = s >= off ? place[s - off] : 0, y = s >= off ? tile[s - off] : 0;
+        __syncthreads();
+        place[s] += x;
+        tile[s] += y;
+        __syncthreads();
+    }
+    const int p0 = place[s] - n, t0 = tile[s] - t;
+    bins[b * kTtBins + s] = p0;
+    for (int k = 0; k < t; ++k)
+        if (t0 + k < maxtiles) tiles[(int64_t)b * maxtiles + t0 + k] = TtTile{s, p0 + 64 * k, n - 64 * k < 64 ? n - 64 * k : 64};
+    if (s == kTtBins - 1) ntiles[b] = tile[s];
+}
+
+// order[b·npts + place] = point, grouped by s (any order within a group)
+__global__ __launch_bounds__(256) void tci_tt_order_kernel(const uint8_t *__restrict__ pts, int64_t npts, int L,
+                                                           int32_t *__restrict__ bins, int32_t *__restrict__ order)
+{
+    __shared__ int32_t h[kTtBins], base[kTtBins];
+    const int b = blockIdx.y;
+    h[threadIdx.x] = 0;
+    __syncthreads();
+    int s[4], r[4];
+    for (int u = 0; u < 4; ++u) {
+        const int64_t q = (int64_t)blockIdx.x * 1024 + u * 256 + threadIdx.x;
+        s[u] = q < npts ? pts[q * L + b] : 0;
+        r[u] = q < npts ? atomicAdd(&h[s[u]], 1) : 0;
+    }
+    __syncthreads();
+    const int n = h[threadIdx.x];
+    base[threadIdx.x] = n ? atomicAdd(&bins[b * kTtBins + threadIdx.x], n) : 0;
+    __syncthreads();
+    for (int u = 0; u < 4; ++u) {
+        const int64_t q = (int64_t)blockIdx.x * 1024 + u * 256 + threadIdx.x;
+        if (q < npts) order[(int64_t)b * npts + base[s[u]] + r[u]] = (int32_t)q;
+    }
+}
+
+// W[q, :] = V[q, :]·T[:, s, :] for the points of one tile (V and W: stride
+// doubles per point, V null: the vector [1]); each sum ascending from 0.0
+template <int J>
+__global__ __launch_bounds__(256) void tci_tt_site_kernel(const double *__restrict__ T, int d0, int d, int d2,
+                                                          const TtTile *__restrict__ tiles,
+                                                          const int32_t *__restrict__ ntiles,
+                                                          const int32_t *__restrict__ order,
+                                                          const double *__restrict__ V, double *__restrict__ W,
+                                                          int stride)
+{
+    extern __shared__ double tile[];   // [i][point], 65 doubles a row (no bank conflicts while staging)
+    if ((int)blockIdx.x >= ntiles[0]) return;
+    const TtTile t = tiles[blockIdx.x];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (int p = wave; p < 64; p += 4) {
+        const int64_t q = order[t.first + (p < t.n ? p : 0)];
+        for (int i = lane; i < d0; i += 64) tile[i * 65 + p] = V ? V[q * stride + i] : 1.0;
+    }
+    __syncthreads();
+    const double *Ts = T + (int64_t)d0 * (t.s - 1);
+    const int64_t cs = (int64_t)d0 * d;   // from one column of the slice to the next
+    const double *v = tile + lane;
+    const int64_t q = order[t.first + (lane < t.n ? lane : 0)];
+    for (int j0 = wave * J; j0 < d2; j0 += 4 * J) {
+        const double *Tj[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) Tj[j] = Ts + cs * (j0 + j < d2 ? j0 + j : d2 - 1);
+        double acc[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) acc[j] = 0.0;
+        int i = 0;
+        for (; i + 4 <= d0; i += 4) {
+            double x[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x[u] = v[(i + u) * 65];
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) acc[j] = acc[j] + x[u] * Tj[j][i + u];
+        }
+        for (; i < d0; ++i) {
+            const double x = v[i * 65];
+#pragma unroll
+            for (int j = 0; j < J; ++j) acc[j] = acc[j] + x * Tj[j][i];
+        }
+        if (lane < t.n) {
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+                if (j0 + j < d2) W[q * stride + j0 + j] = acc[j];
+        }
+    }
+}
+
+// out_tt[q] = V[q·stride]; with fkind also f, and the maxima as in tci_tt_eval_kernel
+__global__ __launch_bounds__(256) void tci_tt_finish_kernel(const double *__restrict__ V, int stride,
+                                                            const uint8_t *__restrict__ pts, int64_t npts, int L,
+                                                            int fkind, const double *__restrict__ params,
+                                                            const int32_t *__restrict__ iparams,
+                                                            double *__restrict__ out_tt, double *__restrict__ out_f,
+                                                            double *__restrict__ blockmax)
+{
+    __shared__ double red[8];
+    const int tid = threadIdx.x;
+    const int64_t q = (int64_t)blockIdx.x * 256 + tid;
+    double le = 0.0, lf = 0.0;
+    if (q < npts) {
+        const double tt = V[q * stride];
+        out_tt[q] = tt;
+        if (fkind) {
+            tci_point x;
+            x.a = pts + q * L;
+            x.b = x.a;
+            x.na = L;
+            x.L = L;
+            const double fv = tci_functor_eval(fkind, params, iparams, &x);
+            if (out_f) out_f[q] = fv;
+            le = fabs(tt - fv);
+            lf = fabs(fv);
+        }
+    }
+    if (!fkind) return;
+    for (int off = 32; off >= 1; off >>= 1) {
+        le = jl_max(le, __shfl_xor(le, off));
+        lf = jl_max(lf, __shfl_xor(lf, off));
+    }
+    if ((tid & 63) == 0) {
+        red[2 * (tid >> 6)] = le;
+        red[2 * (tid >> 6) + 1] = lf;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < 4; ++w) {
+            red[0] = jl_max(red[0], red[2 * w]);
+            red[1] = jl_max(red[1], red[2 * w + 1]);
+        }
+        blockmax[2 * blockIdx.x] = red[0];
+        blockmax[2 * blockIdx.x + 1] = red[1];
+    }
+}
+
+hipError_t launch_tt_group(const uint8_t *pts, int64_t npts, int L, int32_t *bins, TtTile *tiles, int32_t *ntiles,
+                           int maxtiles, int32_t *order, hipStream_t st)
+{
+    const dim3 g((unsigned)((npts + 1023) / 1024), (unsigned)L);
+    hipLaunchKernelGGL(tci_tt_count_kernel, g, dim3(256), 0, st, pts, npts, L, bins);
+    hipLaunchKernelGGL(tci_tt_tiles_kernel, dim3((unsigned)L), dim3(256), 0, st, bins, tiles, ntiles, maxtiles);
+    hipLaunchKernelGGL(tci_tt_order_kernel, g, dim3(256), 0, st, pts, npts, L, bins, order);
+    return hipGetLastError();
+}
+
+hipError_t launch_tt_site(const double *T, int d0, int d, int d2, const TtTile *tiles, const int32_t *ntiles,
+                          int maxtiles, const int32_t *order, const double *V, double *W, int stride, hipStream_t st)
+{
+    const size_t lds = (size_t)d0 * 65 * sizeof(double);
+    // eight columns a wave where there are enough for all four waves
+    const void *k = d2 > 16 ? (const void *)tci_tt_site_kernel<8> : (const void *)tci_tt_site_kernel<4>;
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    if (d2 > 16)
+        hipLaunchKernelGGL((tci_tt_site_kernel<8>), dim3((unsigned)maxtiles), dim3(256), lds, st, T, d0, d, d2, tiles,
+                           ntiles, order, V, W, stride);
+    else
+        hipLaunchKernelGGL((tci_tt_site_kernel<4>), dim3((unsigned)maxtiles), dim3(256), lds, st, T, d0, d, d2, tiles,
+                           ntiles, order, V, W, stride);
+    return hipGetLastError();
+}
+
+hipError_t launch_tt_finish(const double *V, int stride, const uint8_t *pts, int64_t npts, int L, int fkind,
+                            const double *params, const int32_t *iparams, double *out_tt, double *out_f,
+                            double *blockmax, hipStream_t st)
+{
+    hipLaunchKernelGGL(tci_tt_finish_kernel, dim3((unsigned)((npts + 255) / 256)), dim3(256), 0, st, V, stride, pts,
+                       npts, L, fkind, params, iparams, out_tt, out_f, blockmax);
+    return hipGetLastError();
+}
+
 // _floatingzone (globalsearch.jl:43-95) from each start point: one
 // workgroup per point (grid-stride).  Per sweep, the right environments
 // R_b = T_b[:, x_b, :]·R_{b+1} (R_L = [1], each entry summed in ascending
