@@ -85,7 +85,7 @@ struct tci_ctx {
     int rrlu_algo = TCI_RRLU_AUTO;   // factorization kernel of the standalone rrLU
     std::vector<tci_rrlu_tune> tune; // measured AUTO choices (tci_ctx_autotune_rrlu), by side
     int ncu = 0;                     // compute units
-    std::vector<uint8_t> chip_host;  // host copy of the last on-chip rrLU's tables
+    std::vector<uint8_t> chip_host, tile_host;   // host copies of the last rrLU's tables
 };
 
 // a device-to-host copy of a finished result on the context's download
@@ -507,12 +507,6 @@ static tci_status lu_read(tci_ctx *ctx, tci_lu_job *jobs, int64_t count, LuPlan 
     return TCI_OK;
 }
 
-static tci_status lu_plan(tci_ctx *ctx, tci_lu_job *jobs, int64_t count, int64_t tile_budget, LuPlan &P)
-{
-    const tci_status s = lu_read(ctx, jobs, count, P);
-    return s != TCI_OK ? s : lu_partition(ctx, tile_budget, P);
-}
-
 // the tuned entry for a job of largest side s: the first entry at least s,
 // the last one beyond them; null when the context is not tuned
 static const tci_rrlu_tune *tune_for(const tci_ctx *c, int64_t m, int64_t n)
@@ -661,19 +655,15 @@ static void stream_order(const LuPlan &P, std::vector<int32_t> &order)
 
 constexpr int64_t kLuLdsStageCap = 48 * 1024 / 16;   // doubles per staging vector in LDS
 
-tci_status tci_rrlu_batched_f64(tci_ctx *ctx, tci_lu_job *jobs, int64_t count)
+// The launches of a batch whose jobs are known on the host (P.h), jobs their
+// device table.  The tables of each kernel go up from memory of the context: a
+// caller has synchronized the stream since the last call that used it.
+static tci_status lu_launch(tci_ctx *ctx, tci_lu_job *jobs, LuPlan &P)
 {
-    if (!ctx || (!jobs && count > 0) || count < 0) return set_err(TCI_ERR_ARG, "bad arguments");
-    if (count == 0) return TCI_OK;
-    if (count > INT32_MAX) return set_err(TCI_ERR_ARG, "too many jobs");
-    HIPCHK(hipSetDevice(ctx->device));
-    LuPlan P;
-    tci_status ps = lu_plan(ctx, jobs, count, -1, P);
+    const int64_t count = (int64_t)P.h.size();
+    tci_status ps = lu_partition(ctx, -1, P);
     if (ps != TCI_OK) return ps;
     std::vector<int32_t> &tile = P.tile, &stream = P.stream;
-    std::vector<int64_t> &soff = P.soff;
-    const int64_t sc_tot = P.sc_tot;
-    int64_t mx;
     ps = lu_run_chip(ctx, jobs, P, P.chip, 0);
     if (ps != TCI_OK) return ps;
     if (!P.chip.empty() && !P.big.empty()) HIPCHK(hipStreamSynchronize(ctx->stream));   // (chip_host is used again)
@@ -682,25 +672,23 @@ tci_status tci_rrlu_batched_f64(tci_ctx *ctx, tci_lu_job *jobs, int64_t count)
     if (!tile.empty()) {
         uint8_t *d = nullptr;
         const size_t b_idx = lay_align(sizeof(int32_t) * tile.size());
-        const size_t b_off = lay_align(sizeof(int64_t) * soff.size());
-        HIPCHK(hipMallocAsync((void **)&d, b_idx + b_off + sizeof(double) * (size_t)(sc_tot + 1), ctx->stream));
-        hipError_t e = hipMemcpyAsync(d, tile.data(), sizeof(int32_t) * tile.size(), hipMemcpyHostToDevice, ctx->stream);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(d + b_idx, soff.data(), sizeof(int64_t) * soff.size(), hipMemcpyHostToDevice, ctx->stream);
+        const size_t b_off = lay_align(sizeof(int64_t) * P.soff.size());
+        std::vector<uint8_t> &h = ctx->tile_host;
+        h.resize(b_idx + b_off);
+        memcpy(h.data(), tile.data(), sizeof(int32_t) * tile.size());
+        memcpy(h.data() + b_idx, P.soff.data(), sizeof(int64_t) * P.soff.size());
+        HIPCHK(hipMallocAsync((void **)&d, b_idx + b_off + sizeof(double) * (size_t)(P.sc_tot + 1), ctx->stream));
+        hipError_t e = hipMemcpyAsync(d, h.data(), h.size(), hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess)
             e = launch_rrlu_tile(jobs, (const int32_t *)d, (int64_t)tile.size(), (double *)(d + b_idx + b_off),
                                  (const int64_t *)(d + b_idx), ctx->stream);
-        // the host vectors must outlive the copies
-        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
         (void)hipFreeAsync(d, ctx->stream);
         if (e != hipSuccess) return set_err(TCI_ERR_DEVICE, "rrlu tile launch: %s", hipGetErrorString(e));
     }
     if (stream.empty()) return TCI_OK;
-    mx = stream_side(P);
+    const int64_t mx = stream_side(P);
     double *gstage = nullptr;
     if (mx > kLuLdsStageCap) HIPCHK(hipMallocAsync((void **)&gstage, sizeof(double) * 2 * mx * count, ctx->stream));
-    // (the host copy of the order lives in the context: the next call on
-    // this stream synchronizes before it reuses it)
     std::vector<int32_t> &order = ctx->lu_order;
     stream_order(P, order);
     const int64_t ns = (int64_t)order.size();
@@ -713,6 +701,153 @@ tci_status tci_rrlu_batched_f64(tci_ctx *ctx, tci_lu_job *jobs, int64_t count)
     (void)hipFreeAsync(dorder, ctx->stream);
     if (gstage) (void)hipFreeAsync(gstage, ctx->stream);
     if (e != hipSuccess) return set_err(TCI_ERR_DEVICE, "rrlu launch: %s", hipGetErrorString(e));
+    return TCI_OK;
+}
+
+tci_status tci_rrlu_batched_f64(tci_ctx *ctx, tci_lu_job *jobs, int64_t count)
+{
+    if (!ctx || (!jobs && count > 0) || count < 0) return set_err(TCI_ERR_ARG, "bad arguments");
+    if (count == 0) return TCI_OK;
+    if (count > INT32_MAX) return set_err(TCI_ERR_ARG, "too many jobs");
+    HIPCHK(hipSetDevice(ctx->device));
+    LuPlan P;
+    const tci_status ps = lu_read(ctx, jobs, count, P);   // (synchronizes)
+    return ps != TCI_OK ? ps : lu_launch(ctx, jobs, P);
+}
+
+// One matrix from host memory, factored.  A and the job go up together, the
+// factorization and the unpacking of L and U follow without a host round trip
+// (the rank is read on the device), and job, permutations, L and U come down in
+// one copy sized for the largest rank.  For large results, and for luci (left
+// and right of MatrixLUCI instead of L and U), the rank comes down first and then
+// just what it needs.  X: m×p, Y: p×n.
+constexpr size_t kLuOneBytes = (size_t)8 << 20;      // results that come down in one piece
+constexpr size_t kLuStageBytes = (size_t)1 << 20;    // matrices that go up through pinned memory
+
+// columns of `rows` doubles from packed host memory to a caller's buffer
+static void unpack_columns(double *dst, int64_t ld, const double *src, int64_t rows, int64_t cols)
+{
+    if (ld == rows) memcpy(dst, src, sizeof(double) * (size_t)(rows * cols));
+    else
+        for (int64_t j = 0; j < cols; ++j) memcpy(dst + ld * j, src + rows * j, sizeof(double) * (size_t)rows);
+}
+
+static tci_status lu_one(tci_ctx *ctx, const double *A, int64_t lda, int64_t m, int64_t n, int64_t maxrank,
+                         double reltol, double abstol, int32_t leftorth, bool luci, int64_t *rowperm,
+                         int64_t *colperm, double *X, int64_t ldx, double *Y, int64_t ldy, int64_t *npivot,
+                         double *error)
+{
+    HIPCHK(hipSetDevice(ctx->device));
+    hipStream_t st = ctx->stream;
+    const int64_t cap = std::min(std::min(m, n), maxrank);
+    const size_t a_bytes = sizeof(double) * (size_t)(m * n);
+    const size_t b_A = lay_align(a_bytes + 1), b_job = lay_align(sizeof(tci_lu_job));
+    const size_t b_perm = lay_align(sizeof(int32_t) * (size_t)(m + n + 1));
+    const size_t b_lu = sizeof(double) * (size_t)((m + n + 1) * cap);   // L, U, pivots
+    const bool one = !luci && b_lu <= kLuOneBytes;
+    const size_t b_dev = b_A + b_job + b_perm + (one ? b_lu : 0);
+    const bool staged = a_bytes <= kLuStageBytes;
+    const size_t up = (staged ? b_A : 0) + b_job, down = b_job + b_perm + (one ? b_lu : 0);
+    uint8_t *d = nullptr, *d2 = nullptr;
+    PoolBuf host{nullptr, 0};
+    HIPCHK(hipMallocAsync((void **)&d, b_dev, st));
+    hipError_t e = hpool_get(ctx, up > down ? up : down, &host);
+    uint8_t *h = (uint8_t *)host.ptr;
+    uint8_t *djob = d + b_A, *dperm = djob + b_job, *dlu = dperm + b_perm;
+    tci_lu_job j;
+    memset(&j, 0, sizeof j);
+    j.A = (double *)d;
+    j.rowperm = (int32_t *)dperm;
+    j.colperm = (int32_t *)dperm + m;
+    j.m = m;
+    j.n = n;
+    j.maxrank = maxrank;
+    j.reltol = reltol;
+    j.abstol = abstol;
+    j.leftorth = leftorth ? 1 : 0;
+    if (e == hipSuccess && staged) {
+        for (int64_t q = 0; q < n && m > 0; ++q)
+            memcpy(h + sizeof(double) * (size_t)(m * q), A + lda * q, sizeof(double) * (size_t)m);
+        memcpy(h + b_A, &j, sizeof j);
+        e = hipMemcpyAsync(d, h, b_A + b_job, hipMemcpyHostToDevice, st);
+    } else if (e == hipSuccess) {
+        memcpy(h, &j, sizeof j);
+        e = hipMemcpyAsync(djob, h, b_job, hipMemcpyHostToDevice, st);
+        if (e == hipSuccess && lda == m) e = hipMemcpyAsync(d, A, a_bytes, hipMemcpyHostToDevice, st);
+        else if (e == hipSuccess)
+            e = hipMemcpy2DAsync(d, sizeof(double) * m, A, sizeof(double) * lda, sizeof(double) * m, n,
+                                 hipMemcpyHostToDevice, st);
+    }
+    LuPlan P;
+    P.h.assign(1, j);
+    P.mx = m > n ? m : n;
+    tci_status s = TCI_OK;
+    if (e == hipSuccess) s = lu_launch(ctx, (tci_lu_job *)djob, P);
+    double *dL = (double *)dlu;
+    if (e == hipSuccess && s == TCI_OK && one)
+        // (U starts where L of the rank found ends: the kernel packs them)
+        e = launch_lu_unpack((const tci_lu_job *)djob, (m + n + 1) * cap, dL, nullptr, nullptr, nullptr, st);
+    if (e == hipSuccess && s == TCI_OK) e = hipMemcpyAsync(h, djob, down, hipMemcpyDeviceToHost, st);
+    const hipError_t es = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = es;
+    if (e == hipSuccess && s == TCI_OK) {
+        memcpy(&j, h, sizeof j);
+        const int64_t p = j.npivot;
+        const int32_t *perm = (const int32_t *)(h + b_job);
+        for (int64_t i = 0; i < m; ++i) rowperm[i] = perm[i];
+        for (int64_t q = 0; q < n; ++q) colperm[q] = perm[m + q];
+        *npivot = p;
+        *error = j.error;
+        const size_t nl = (size_t)(m * p), nu = (size_t)(p * n);
+        if (p > 0 && one) {
+            const double *lu = (const double *)(h + b_job + b_perm);
+            unpack_columns(X, ldx, lu, m, p);
+            unpack_columns(Y, ldy, lu + nl, p, n);
+        } else if (p > 0 && (!luci || j.status == TCI_OK)) {
+            // L, U, the pivots and U11 transposed; for luci also left and right
+            const size_t nt = luci && !leftorth && p <= kLuciSolveMax ? (size_t)(p * p) : 0;
+            const size_t tot = nl + nu + (size_t)p + nt + (luci ? nl + nu : 0);
+            e = hipMallocAsync((void **)&d2, sizeof(double) * tot, st);
+            double *L = (double *)d2, *U = L + nl, *diag = U + nu, *UT = diag + p, *x = luci ? UT + nt : L,
+                   *y = luci ? x + nl : U;
+            if (e == hipSuccess)
+                e = launch_lu_unpack((const tci_lu_job *)djob, (m + n + 1) * p, L, U, diag,
+                                     nt ? UT : nullptr, st);
+            if (e == hipSuccess && luci)
+                e = launch_luci(m, n, p, j.leftorth, (int32_t *)dperm, (int32_t *)dperm + m, L, U, UT, x, m, y, p, st);
+            const size_t bx = sizeof(double) * nl, by = sizeof(double) * nu;
+            if (bx + by <= kLuOneBytes) {
+                PoolBuf h2{nullptr, 0};
+                if (e == hipSuccess) e = hpool_get(ctx, bx + by, &h2);
+                if (e == hipSuccess) e = hipMemcpyAsync(h2.ptr, x, bx + by, hipMemcpyDeviceToHost, st);
+                if (e == hipSuccess) e = hipStreamSynchronize(st);
+                if (e == hipSuccess) {
+                    unpack_columns(X, ldx, (const double *)h2.ptr, m, p);
+                    unpack_columns(Y, ldy, (const double *)h2.ptr + nl, p, n);
+                }
+                if (h2.ptr) hpool_put(ctx, h2);
+            } else {
+                const auto get = [&](double *dst, int64_t ld, const double *src, int64_t rows, int64_t cols) {
+                    return ld == rows ? hipMemcpyAsync(dst, src, sizeof(double) * (size_t)(rows * cols),
+                                                       hipMemcpyDeviceToHost, st)
+                                      : hipMemcpy2DAsync(dst, sizeof(double) * (size_t)ld, src,
+                                                         sizeof(double) * (size_t)rows, sizeof(double) * (size_t)rows,
+                                                         (size_t)cols, hipMemcpyDeviceToHost, st);
+                };
+                if (e == hipSuccess) e = get(X, ldx, x, m, p);
+                if (e == hipSuccess) e = get(Y, ldy, y, p, n);
+                if (e == hipSuccess) e = hipStreamSynchronize(st);
+            }
+        }
+    }
+    (void)hipFreeAsync(d, st);
+    if (d2) (void)hipFreeAsync(d2, st);
+    if (host.ptr) hpool_put(ctx, host);
+    if (s != TCI_OK) return s;
+    if (e != hipSuccess) return set_err(TCI_ERR_DEVICE, "rrlu: %s", hipGetErrorString(e));
+    if (j.status == TCI_ERR_NAN_L) return set_err(TCI_ERR_NAN_L, "lu.L contains NaNs");
+    if (j.status == TCI_ERR_NAN_U) return set_err(TCI_ERR_NAN_U, "lu.U contains NaNs");
+    if (j.status != TCI_OK) return set_err((tci_status)j.status, "rrlu failed");
     return TCI_OK;
 }
 
@@ -926,58 +1061,8 @@ tci_status tci_rrlu_f64(tci_ctx *ctx, const double *A, int64_t lda, int64_t m, i
     if ((cap > 0 && m > 0 && (!Lh || ldl < m)) || (cap > 0 && n > 0 && (!Uh || ldu < cap)))
         return set_err(TCI_ERR_ARG, "L/U buffers too small");
     if (m * n > ((int64_t)1 << 31)) return set_err(TCI_ERR_ARG, "matrix too large");
-    HIPCHK(hipSetDevice(ctx->device));
-    hipStream_t st = ctx->stream;
-    const size_t mn = (size_t)(m * n);
-    double *dA = nullptr, *dL = nullptr, *dU = nullptr;
-    int32_t *dperm = nullptr;
-    tci_lu_job *dj = nullptr;
-    HIPCHK(hipMallocAsync((void **)&dA, sizeof(double) * (mn ? mn : 1), st));
-    HIPCHK(hipMallocAsync((void **)&dperm, sizeof(int32_t) * (size_t)(m + n + 1), st));
-    HIPCHK(hipMallocAsync((void **)&dj, sizeof(tci_lu_job), st));
-    if (mn) HIPCHK(hipMemcpy2DAsync(dA, sizeof(double) * m, A, sizeof(double) * lda, sizeof(double) * m,
-                                    n, hipMemcpyHostToDevice, st));
-    tci_lu_job j;
-    memset(&j, 0, sizeof j);
-    j.A = dA;
-    j.rowperm = dperm;
-    j.colperm = dperm + m;
-    j.m = m;
-    j.n = n;
-    j.maxrank = maxrank;
-    j.reltol = reltol;
-    j.abstol = abstol;
-    j.leftorth = leftorth ? 1 : 0;
-    HIPCHK(hipMemcpyAsync(dj, &j, sizeof j, hipMemcpyHostToDevice, st));
-    tci_status s = tci_rrlu_batched_f64(ctx, dj, 1);
-    if (s != TCI_OK) return s;
-    HIPCHK(hipMemcpyAsync(&j, dj, sizeof j, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    const int64_t p = j.npivot;
-    if (p > 0) {
-        HIPCHK(hipMallocAsync((void **)&dL, sizeof(double) * (size_t)(m * p + 1), st));
-        HIPCHK(hipMallocAsync((void **)&dU, sizeof(double) * (size_t)(p * n + 1), st));
-        HIPCHK(launch_lu_unpack(dA, m, n, p, j.leftorth, dL, m, dU, p, st));
-        HIPCHK(hipMemcpy2DAsync(Lh, sizeof(double) * ldl, dL, sizeof(double) * m, sizeof(double) * m, p,
-                                hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpy2DAsync(Uh, sizeof(double) * ldu, dU, sizeof(double) * p, sizeof(double) * p, n,
-                                hipMemcpyDeviceToHost, st));
-    }
-    std::vector<int32_t> perm((size_t)(m + n + 1));
-    HIPCHK(hipMemcpyAsync(perm.data(), dperm, sizeof(int32_t) * (size_t)(m + n), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    for (int64_t i = 0; i < m; ++i) rowperm[i] = perm[(size_t)i];
-    for (int64_t q = 0; q < n; ++q) colperm[q] = perm[(size_t)(m + q)];
-    (void)hipFreeAsync(dA, st);
-    (void)hipFreeAsync(dperm, st);
-    (void)hipFreeAsync(dj, st);
-    if (dL) (void)hipFreeAsync(dL, st);
-    if (dU) (void)hipFreeAsync(dU, st);
-    *npivot = p;
-    *error = j.error;
-    if (j.status == TCI_ERR_NAN_L) return set_err(TCI_ERR_NAN_L, "lu.L contains NaNs");
-    if (j.status == TCI_ERR_NAN_U) return set_err(TCI_ERR_NAN_U, "lu.U contains NaNs");
-    return TCI_OK;
+    return lu_one(ctx, A, lda, m, n, maxrank, reltol, abstol, leftorth, false, rowperm, colperm, Lh, ldl, Uh, ldu,
+                  npivot, error);
 }
 
 tci_status tci_luci_f64(tci_ctx *ctx, const double *A, int64_t lda, int64_t m, int64_t n, int64_t maxrank,
@@ -994,60 +1079,8 @@ tci_status tci_luci_f64(tci_ctx *ctx, const double *A, int64_t lda, int64_t m, i
     if ((cap > 0 && m > 0 && (!left || ldleft < m)) || (cap > 0 && n > 0 && (!right || ldright < cap)))
         return set_err(TCI_ERR_ARG, "left/right buffers too small");
     if (m * n > ((int64_t)1 << 31)) return set_err(TCI_ERR_ARG, "matrix too large");
-    HIPCHK(hipSetDevice(ctx->device));
-    hipStream_t st = ctx->stream;
-    const size_t mn = (size_t)(m * n);
-    double *dA = nullptr, *dLU = nullptr;
-    int32_t *dperm = nullptr;
-    tci_lu_job *dj = nullptr;
-    HIPCHK(hipMallocAsync((void **)&dA, sizeof(double) * (mn ? mn : 1), st));
-    HIPCHK(hipMallocAsync((void **)&dperm, sizeof(int32_t) * (size_t)(m + n + 1), st));
-    HIPCHK(hipMallocAsync((void **)&dj, sizeof(tci_lu_job), st));
-    if (mn) HIPCHK(hipMemcpy2DAsync(dA, sizeof(double) * m, A, sizeof(double) * lda, sizeof(double) * m, n,
-                                    hipMemcpyHostToDevice, st));
-    tci_lu_job j;
-    memset(&j, 0, sizeof j);
-    j.A = dA;
-    j.rowperm = dperm;
-    j.colperm = dperm + m;
-    j.m = m;
-    j.n = n;
-    j.maxrank = maxrank;
-    j.reltol = reltol;
-    j.abstol = abstol;
-    j.leftorth = leftorth ? 1 : 0;
-    HIPCHK(hipMemcpyAsync(dj, &j, sizeof j, hipMemcpyHostToDevice, st));
-    tci_status s = tci_rrlu_batched_f64(ctx, dj, 1);
-    if (s != TCI_OK) return s;
-    HIPCHK(hipMemcpyAsync(&j, dj, sizeof j, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    const int64_t p = j.npivot;
-    if (j.status == TCI_OK && p > 0) {
-        // unpacked L, U, then left and right (device), then host copies
-        const size_t nl = (size_t)(m * p), nu = (size_t)(p * n);
-        HIPCHK(hipMallocAsync((void **)&dLU, sizeof(double) * (2 * (nl + nu) + 1), st));
-        double *dL = dLU, *dU = dLU + nl, *dleft = dU + nu, *dright = dleft + nl;
-        HIPCHK(launch_lu_unpack(dA, m, n, p, j.leftorth, dL, m, dU, p, st));
-        HIPCHK(launch_luci(m, n, p, j.leftorth, dperm, dperm + m, dL, dU, dleft, m, dright, p, st));
-        HIPCHK(hipMemcpy2DAsync(left, sizeof(double) * ldleft, dleft, sizeof(double) * m, sizeof(double) * m, p,
-                                hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpy2DAsync(right, sizeof(double) * ldright, dright, sizeof(double) * p, sizeof(double) * p, n,
-                                hipMemcpyDeviceToHost, st));
-    }
-    std::vector<int32_t> perm((size_t)(m + n + 1));
-    HIPCHK(hipMemcpyAsync(perm.data(), dperm, sizeof(int32_t) * (size_t)(m + n), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    for (int64_t i = 0; i < m; ++i) rowperm[i] = perm[(size_t)i];
-    for (int64_t q = 0; q < n; ++q) colperm[q] = perm[(size_t)(m + q)];
-    (void)hipFreeAsync(dA, st);
-    (void)hipFreeAsync(dperm, st);
-    (void)hipFreeAsync(dj, st);
-    if (dLU) (void)hipFreeAsync(dLU, st);
-    *npivot = p;
-    *error = j.error;
-    if (j.status == TCI_ERR_NAN_L) return set_err(TCI_ERR_NAN_L, "lu.L contains NaNs");
-    if (j.status == TCI_ERR_NAN_U) return set_err(TCI_ERR_NAN_U, "lu.U contains NaNs");
-    return TCI_OK;
+    return lu_one(ctx, A, lda, m, n, maxrank, reltol, abstol, leftorth, true, rowperm, colperm, left, ldleft, right,
+                  ldright, npivot, error);
 }
 
 tci_status tci_gemm_f64(tci_ctx *ctx, int64_t M, int64_t N, int64_t K, const double *A, int64_t lda,
@@ -1094,11 +1127,18 @@ struct TtDevice {
     std::vector<int64_t> off;   // slot of each site in `cores` (doubles)
     int64_t maxsite = 0, maxside = 0;
     uint8_t *arena = nullptr;
-    double *cores = nullptr, *wl = nullptr, *wu = nullptr, *wc = nullptr, *wp = nullptr, *diag = nullptr;
+    double *cores = nullptr, *wl = nullptr, *wu = nullptr, *wc = nullptr, *wp = nullptr, *wt = nullptr, *diag = nullptr;
     int32_t *perm = nullptr;
     tci_lu_job *job = nullptr;
+    size_t res_bytes = 0;        // job, pivots and permutations, in this order
+    uint8_t *hres = nullptr;     // their host copy (pinned)
+    PoolBuf hbuf{nullptr, 0};
     ~TtDevice()
     {
+        if (hbuf.ptr) {
+            (void)hipStreamSynchronize(ctx->stream);
+            hpool_put(ctx, hbuf);
+        }
         if (arena) (void)hipFreeAsync(arena, ctx->stream);
     }
 };
@@ -1137,12 +1177,17 @@ static tci_status tt_upload(tci_ctx *ctx, TtDevice &T, int32_t L, const int64_t 
         const int64_t side = (s1 > s2 ? s1 : s2) + T.links[(size_t)b] + T.links[(size_t)b + 1];
         T.maxside = side > T.maxside ? side : T.maxside;
     }
-    // cores | L | U | carried factor | product | diagonal | perm | job
+    // cores | L | U | carried factor | product | U11 transposed | job | diagonal | perm
     const size_t b_cores = lay_align(sizeof(double) * (size_t)tot);
     const size_t b_w = lay_align(sizeof(double) * (size_t)T.maxsite);
     const size_t b_diag = lay_align(sizeof(double) * (size_t)T.maxside);
     const size_t b_perm = lay_align(sizeof(int32_t) * (size_t)T.maxside);
-    const size_t bytes = b_cores + 4 * b_w + b_diag + b_perm + lay_align(sizeof(tci_lu_job));
+    const size_t b_job = lay_align(sizeof(tci_lu_job));
+    const size_t b_t = lay_align(sizeof(double) * (size_t)std::min(T.maxsite, kLuciSolveMax * kLuciSolveMax));
+    const size_t bytes = b_cores + 4 * b_w + b_t + b_diag + b_perm + b_job;
+    T.res_bytes = b_job + b_diag + b_perm;
+    HIPCHK(hpool_get(ctx, T.res_bytes, &T.hbuf));
+    T.hres = (uint8_t *)T.hbuf.ptr;
     HIPCHK(hipMallocAsync((void **)&T.arena, bytes, ctx->stream));
     uint8_t *p = T.arena;
     T.cores = (double *)p;
@@ -1155,11 +1200,13 @@ static tci_status tt_upload(tci_ctx *ctx, TtDevice &T, int32_t L, const int64_t 
     p += b_w;
     T.wp = (double *)p;
     p += b_w;
+    T.wt = (double *)p;
+    p += b_t;
+    T.job = (tci_lu_job *)p;
+    p += b_job;
     T.diag = (double *)p;
     p += b_diag;
     T.perm = (int32_t *)p;
-    p += b_perm;
-    T.job = (tci_lu_job *)p;
     HIPCHK(hipMemcpyAsync(T.cores, cores, sizeof(double) * (size_t)tot, hipMemcpyHostToDevice, ctx->stream));
     return TCI_OK;
 }
@@ -1185,9 +1232,11 @@ static tci_status tt_download(TtDevice &T, int64_t *linkdims, double *cores)
 // replaced by one of them and the other multiplied into the neighbour.
 // The whole sweep in one workgroup (launch_tt_sweep) for trains whose every
 // bond matrix holds at most kTtFusedElems entries: there the host-driven
-// sweep spends its time in per-bond round trips (about 0.3 ms each), not in
-// the factorizations.  Same operations per entry, so the same bits.
-constexpr int64_t kTtFusedElems = (int64_t)256 * 256;
+// sweep spends its time in per-bond round trips (about 80 us each), not in
+// the factorizations.  Same operations per entry, so the same bits.  Measured
+// (compress! of 20 sites, one workgroup / bond by bond, ms): 1024 entries 2.8 /
+// 3.3, 2304 4.5 / 5.3, 4096 7.3 / 6.1, 9216 15 / 7.5, 62 208 130 / 14.
+constexpr int64_t kTtFusedElems = 3072;
 constexpr int64_t kTtStageCap = 48 * 1024 / 16;   // doubles per LDS staging vector
 constexpr int64_t kTtMatCap = 96 * 1024 / 8;       // doubles of LDS for a bond matrix
 
@@ -1283,8 +1332,8 @@ static tci_status tt_sweep(TtDevice &T, int32_t method, int32_t forward, int64_t
     if (pivoterrors)
         for (int64_t k = 0; k <= R; ++k) pivoterrors[k] = 0.0;
     std::vector<std::vector<int32_t>> piv((size_t)(L > 1 ? L - 1 : 0));
-    std::vector<int32_t> hperm((size_t)T.maxside);
-    std::vector<double> hdiag((size_t)T.maxside);
+    const double *hdiag = (const double *)(T.hres + ((uint8_t *)T.diag - (uint8_t *)T.job));
+    const int32_t *hperm = (const int32_t *)(T.hres + ((uint8_t *)T.perm - (uint8_t *)T.job));
     for (int i = 0; i < L - 1; ++i) {
         const int b = forward ? i : L - 2 - i;
         const int s = forward ? b : b + 1;
@@ -1302,28 +1351,31 @@ static tci_status tt_sweep(TtDevice &T, int32_t method, int32_t forward, int64_t
         j.reltol = reltol;
         j.abstol = abstol;
         j.leftorth = forward ? 1 : 0;
-        HIPCHK(hipMemcpyAsync(T.job, &j, sizeof j, hipMemcpyHostToDevice, st));
-        tci_status ls = tci_rrlu_batched_f64(ctx, T.job, 1);
+        memcpy(T.hres, &j, sizeof j);
+        HIPCHK(hipMemcpyAsync(T.job, T.hres, sizeof j, hipMemcpyHostToDevice, st));
+        LuPlan P;
+        P.h.assign(1, j);
+        P.mx = m > n ? m : n;
+        tci_status ls = lu_launch(ctx, T.job, P);
         if (ls != TCI_OK) return ls;
-        // the pivots are the diagonal of the factored matrix
-        const int64_t mn = m < n ? m : n;
-        HIPCHK(hipMemcpyAsync(&j, T.job, sizeof j, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpy2DAsync(hdiag.data(), sizeof(double), A, sizeof(double) * (size_t)(m + 1), sizeof(double),
-                                (size_t)mn, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(hperm.data(), T.perm, sizeof(int32_t) * (size_t)(m + n), hipMemcpyDeviceToHost, st));
+        // L, U and the pivots, the rank read on the device; then job, pivots and
+        // permutations in one copy (they lie next to each other)
+        HIPCHK(launch_lu_unpack(T.job, (m + n + 1) * std::min(m, n), T.wl, T.wu, T.diag,
+                                method == 1 && !forward ? T.wt : nullptr, st));
+        HIPCHK(hipMemcpyAsync(T.hres, T.job, T.res_bytes, hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
+        memcpy(&j, T.hres, sizeof j);
         if (j.status == TCI_ERR_NAN_L) return set_err(TCI_ERR_NAN_L, "lu.L contains NaNs");
         if (j.status == TCI_ERR_NAN_U) return set_err(TCI_ERR_NAN_U, "lu.U contains NaNs");
         if (j.status != TCI_OK) return set_err((tci_status)j.status, "rrlu failed at bond %d", b + 1);
         const int64_t p = j.npivot;
-        HIPCHK(launch_lu_unpack(A, m, n, p, j.leftorth, T.wl, m, T.wu, p, st));
         // forward: the site takes left (m×p), right goes to wc; backward:
         // the site takes right (p×n), left goes to wc
         double *lft = forward ? A : T.wc, *rgt = forward ? T.wc : A;
         if (method == 0)
             HIPCHK(launch_lu_permute(m, n, p, T.perm, T.perm + m, T.wl, T.wu, lft, m, rgt, p, st));
         else
-            HIPCHK(launch_luci(m, n, p, j.leftorth, T.perm, T.perm + m, T.wl, T.wu, lft, m, rgt, p, st));
+            HIPCHK(launch_luci(m, n, p, j.leftorth, T.perm, T.perm + m, T.wl, T.wu, T.wt, lft, m, rgt, p, st));
         if (forward) {
             // site b+1 ← right · (χ_{b+1} × d_{b+1} χ_{b+2})
             const int64_t nn = T.d[(size_t)b + 1] * T.links[(size_t)b + 2];
@@ -1338,10 +1390,10 @@ static tci_status tt_sweep(TtDevice &T, int32_t method, int32_t forward, int64_t
             HIPCHK(hipMemcpyAsync(pv, T.wp, sizeof(double) * (size_t)(mm * p), hipMemcpyDeviceToDevice, st));
         }
         T.links[(size_t)b + 1] = p;
-        piv[(size_t)b].assign(hperm.data(), hperm.data() + p);
-        piv[(size_t)b].insert(piv[(size_t)b].end(), hperm.data() + m, hperm.data() + m + p);
+        piv[(size_t)b].assign(hperm, hperm + p);
+        piv[(size_t)b].insert(piv[(size_t)b].end(), hperm + m, hperm + m + p);
         if (pivoterrors) {
-            for (int64_t k = 0; k < p; ++k) pivoterrors[k] = nan_max(pivoterrors[k], fabs(hdiag[(size_t)k]));
+            for (int64_t k = 0; k < p; ++k) pivoterrors[k] = nan_max(pivoterrors[k], fabs(hdiag[k]));
             pivoterrors[p] = nan_max(pivoterrors[p], j.error);
         }
     }

@@ -125,16 +125,21 @@ hipError_t launch_tt_sweep(const TtSweepArgs &a, hipStream_t st);
 hipError_t launch_gemm(int64_t M, int64_t N, int64_t K, const double *A, int64_t lda, const double *B, int64_t ldb,
                        double *Cm, int64_t ldc, hipStream_t st);
 // left(luci) (m×p, ld ldl) and right(luci) (p×n, ld ldr) of MatrixLUCI from
-// the unpacked L (m×p) and U (p×n) and the 1-based permutations
+// the unpacked L (m×p) and U (p×n), U11 transposed (p×p, needed without leftorth
+// up to kLuciSolveMax) and the 1-based permutations
+constexpr int64_t kLuciSolveMax = 256;   // 128 KiB of LDS
 hipError_t launch_luci(int64_t m, int64_t n, int64_t p, int leftorth, const int32_t *rowperm, const int32_t *colperm,
-                       const double *L, const double *U, double *left, int64_t ldl, double *right, int64_t ldr,
-                       hipStream_t st);
+                       const double *L, const double *U, const double *UT, double *left, int64_t ldl, double *right,
+                       int64_t ldr, hipStream_t st);
 // left(lu)/right(lu) with the permutations applied, from the unpacked L, U
 hipError_t launch_lu_permute(int64_t m, int64_t n, int64_t p, const int32_t *rowperm, const int32_t *colperm,
                              const double *L, const double *U, double *left, int64_t ldl, double *right, int64_t ldr,
                              hipStream_t st);
-hipError_t launch_lu_unpack(const double *A, int64_t m, int64_t n, int64_t p, int leftorth,
-                            double *L, int64_t ldl, double *U, int64_t ldu, hipStream_t st);
+// the factors of a finished job (its rank is read on the device): L m×p and U p×n
+// with leading dimensions m and p (U null: right behind L), diag the p pivots and
+// UT U11 transposed, p×p (null: not wanted); most: an upper bound of (m + n + 1)·p
+hipError_t launch_lu_unpack(const tci_lu_job *job, int64_t most, double *L, double *U, double *diag, double *UT,
+                            hipStream_t st);
 hipError_t launch_kron_center(const uint8_t *left, int64_t nI, int nl, const int32_t *cdims, int M,
                               int64_t nc, uint8_t *rowsx, int stride, hipStream_t st);
 int eval_blocks(int64_t tot);

@@ -14,6 +14,8 @@
 // reduction costs one barrier.  Compiled with -ffp-contract=off.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "tci_devteam.h"
 #include "tci_engine.h"
 #include "tci_kernels.h"
@@ -399,14 +401,32 @@ __device__ __forceinline__ void lu_unpack_at(int64_t q, const double *A, int64_t
     }
 }
 
-__global__ void tci_lu_unpack_kernel(const double *__restrict__ A, int64_t m, int64_t n, int64_t p,
-                                     int leftorth, double *__restrict__ L, int64_t ldl,
-                                     double *__restrict__ U, int64_t ldu)
+// The factors of a finished job, whose rank is read where it lies (no host round
+// trip before this launch): L m×p and U p×n (null: right behind L), the pivots in
+// diag unless null, and with UT non-null the p×p block U11 transposed (for ranks
+// up to kLuciSolveMax)
+__global__ __launch_bounds__(256) void tci_lu_unpack_kernel(const tci_lu_job *__restrict__ job, double *__restrict__ L,
+                                                            double *__restrict__ U, double *__restrict__ diag,
+                                                            double *__restrict__ UT)
 {
+    const double *A = job->A;
+    const int64_t m = job->m, n = job->n, p = job->npivot;
+    const int leftorth = job->leftorth;
     const int64_t nl = m * p, nu = p * n;
-    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < nl + nu;
-         q += (int64_t)gridDim.x * blockDim.x)
-        lu_unpack_at(q, A, m, p, leftorth, L, ldl, U, ldu);
+    if (!U) U = L + nl;
+    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < nl + nu + p;
+         q += (int64_t)gridDim.x * blockDim.x) {
+        if (q >= nl + nu) {
+            const int64_t k = q - nl - nu;
+            if (diag) diag[k] = A[k + m * k];
+            continue;
+        }
+        lu_unpack_at(q, A, m, p, leftorth, L, m, U, p);
+        if (UT && p <= kLuciSolveMax && q >= nl && q - nl < p * p) {
+            const int64_t r = q - nl, j = r / p, i = r - j * p;
+            UT[j + p * i] = U[r];
+        }
+    }
 }
 
 // ------------------------------------------------------------ products
@@ -422,20 +442,53 @@ __device__ __forceinline__ void gemm_at(int64_t q, int64_t M, int64_t K, const d
     Cm[i + ldc * j] = acc;
 }
 
-__global__ void tci_gemm_kernel(int64_t M, int64_t N, int64_t K, const double *__restrict__ A, int64_t lda,
-                                const double *__restrict__ B, int64_t ldb, double *__restrict__ Cm, int64_t ldc)
+// A workgroup forms a 32×32 block of C, four entries a thread, from LDS copies of
+// 16 columns of A and rows of B at a time (one thread per entry with both factors
+// read from memory took 38 us for 2048 x 128 times 128 x 128, this 21 us; the
+// library's matrix product fuses the rounding that the reference's values have)
+constexpr int kGemmTile = 32, kGemmK = 16;
+__global__ __launch_bounds__(256) void tci_gemm_kernel(int64_t M, int64_t N, int64_t K, const double *__restrict__ A,
+                                                       int64_t lda, const double *__restrict__ B, int64_t ldb,
+                                                       double *__restrict__ Cm, int64_t ldc)
 {
-    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < M * N;
-         q += (int64_t)gridDim.x * blockDim.x)
-        gemm_at(q, M, K, A, lda, B, ldb, Cm, ldc);
+    __shared__ double sa[kGemmK][kGemmTile], sb[kGemmTile][kGemmK + 1];
+    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    const int64_t mt = (M + kGemmTile - 1) / kGemmTile, nt = (N + kGemmTile - 1) / kGemmTile;
+    for (int64_t t = blockIdx.x; t < mt * nt; t += gridDim.x) {
+        const int64_t i0 = (t % mt) * kGemmTile, j0 = (t / mt) * kGemmTile;
+        double acc[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
+        for (int64_t k0 = 0; k0 < K; k0 += kGemmK) {
+            const int kn = (int)(K - k0 < kGemmK ? K - k0 : kGemmK);
+            for (int q = threadIdx.x; q < kGemmK * kGemmTile; q += 256) {
+                const int i = q % kGemmTile, k = q / kGemmTile;
+                sa[k][i] = k < kn && i0 + i < M ? A[i0 + i + lda * (k0 + k)] : 0.0;
+                const int kk = q % kGemmK, j = q / kGemmK;
+                sb[j][kk] = kk < kn && j0 + j < N ? B[k0 + kk + ldb * (j0 + j)] : 0.0;
+            }
+            __syncthreads();
+            // (no padded terms: they could turn a sum of -0 or an infinity)
+            for (int k = 0; k < kn; ++k)
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int w = 0; w < 2; ++w) acc[u][w] = acc[u][w] + sa[k][tx + 16 * u] * sb[ty + 16 * w][k];
+            __syncthreads();
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+                const int64_t i = i0 + tx + 16 * u, j = j0 + ty + 16 * w;
+                if (i < M && j < N) Cm[i + ldc * j] = acc[u][w];
+            }
+    }
 }
 
 hipError_t launch_gemm(int64_t M, int64_t N, int64_t K, const double *A, int64_t lda, const double *B, int64_t ldb,
                        double *Cm, int64_t ldc, hipStream_t st)
 {
-    const int64_t tot = M * N;
-    if (tot == 0) return hipSuccess;
-    int64_t blocks = (tot + 255) / 256;
+    if (M * N == 0) return hipSuccess;
+    int64_t blocks = ((M + kGemmTile - 1) / kGemmTile) * ((N + kGemmTile - 1) / kGemmTile);
     if (blocks > 65535) blocks = 65535;
     hipLaunchKernelGGL(tci_gemm_kernel, dim3((unsigned)blocks), dim3(256), 0, st, M, N, K, A, lda, B, ldb, Cm, ldc);
     return hipGetLastError();
@@ -502,6 +555,71 @@ __device__ __forceinline__ void luci_at(int64_t q, int64_t m, int64_t p, int lef
     }
 }
 
+// The standalone kernels split the two factors.  A product's entries are
+// independent, one thread each.  A substitution is a chain of p²/2 dependent
+// subtractions per row whatever is done, so a wave runs 64 rows side by side with
+// their solved entries in LDS and the triangular factor read through scalar loads
+// (one thread per row, its own outputs read back from memory, took up to 527 us
+// for 864 x 72; these 68).
+
+// left = colmatrix (L·U[:,1:p], m×p) or right = rowmatrix (L[1:p,:]·U, p×n), by leftorth
+__global__ __launch_bounds__(256) void tci_luci_product_kernel(int64_t m, int64_t n, int64_t p, int leftorth,
+                                                               const int32_t *__restrict__ rowperm,
+                                                               const int32_t *__restrict__ colperm,
+                                                               const double *__restrict__ L,
+                                                               const double *__restrict__ U, double *__restrict__ left,
+                                                               int64_t ldl, double *__restrict__ right, int64_t ldr)
+{
+    const int64_t rows = leftorth ? p : m, cols = leftorth ? n : p;
+    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < rows * cols;
+         q += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t j = q / rows, i = q - j * rows;
+        int64_t tmax = i < j ? i : j;
+        if (tmax > p - 1) tmax = p - 1;
+        double s = 0.0;
+        for (int64_t t = 0; t <= tmax; ++t) s = s + L[i + m * t] * U[t + p * j];
+        if (leftorth) right[i + ldr * (colperm[j] - 1)] = s;
+        else left[(rowperm[i] - 1) + ldl * j] = s;
+    }
+}
+
+// left = colstimespivotinv ([I; L21·L11⁻¹], leftorth) or right = pivotinvtimesrows
+// ([I U11⁻¹·U12]).  Vector v (row v of left, column v of right) is a unit vector
+// for v < p; else x_j = b_j - Σ_{t>j} x_t·M[t, j] with M = L11, or U11 transposed
+// (unit diagonals), j descending, each sum in ascending t.
+__global__ __launch_bounds__(64) void tci_luci_solve_kernel(int64_t nv, int64_t m, int p, int leftorth,
+                                                            const int32_t *__restrict__ perm,
+                                                            const double *__restrict__ LU,
+                                                            const double *__restrict__ M, int64_t ldm,
+                                                            double *__restrict__ out, int64_t ldo)
+{
+    extern __shared__ double x[];   // [entry][vector]
+    const int lane = threadIdx.x;
+    const int64_t v = (int64_t)blockIdx.x * 64 + lane;
+    const bool have = v < nv;
+    const int64_t vc = have ? v : nv - 1, at = perm[vc] - 1;
+    // entry j of vector v: b[bs·j], out[os·j]
+    const double *b = leftorth ? LU + vc : LU + (int64_t)p * vc;
+    const int64_t bs = leftorth ? m : 1, os = leftorth ? ldo : 1;
+    double *o = leftorth ? out + at : out + ldo * at;
+    for (int j = p - 1; j >= 0; --j) {
+        const double *Mj = M + ldm * j;
+        double s = b[bs * j];
+        int t = j + 1;
+        for (; t + 8 <= p; t += 8) {
+            double y[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) y[u] = x[(t + u) * 64 + lane] * Mj[t + u];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s = s - y[u];
+        }
+        for (; t < p; ++t) s = s - x[t * 64 + lane] * Mj[t];
+        x[j * 64 + lane] = s;   // (the diagonal is 1)
+        if (have) o[os * j] = v < p ? (v == j ? 1.0 : 0.0) : s;
+    }
+}
+
+// one thread per row of left and column of right: ranks beyond the solve kernel's LDS
 __global__ void tci_luci_kernel(int64_t m, int64_t n, int64_t p, int leftorth, const int32_t *__restrict__ rowperm,
                                 const int32_t *__restrict__ colperm, const double *__restrict__ L,
                                 const double *__restrict__ U, double *__restrict__ left, int64_t ldl,
@@ -513,11 +631,29 @@ __global__ void tci_luci_kernel(int64_t m, int64_t n, int64_t p, int leftorth, c
 }
 
 hipError_t launch_luci(int64_t m, int64_t n, int64_t p, int leftorth, const int32_t *rowperm, const int32_t *colperm,
-                       const double *L, const double *U, double *left, int64_t ldl, double *right, int64_t ldr,
-                       hipStream_t st)
+                       const double *L, const double *U, const double *UT, double *left, int64_t ldl, double *right,
+                       int64_t ldr, hipStream_t st)
 {
     const int64_t tot = m + n;
     if (tot == 0 || p == 0) return hipSuccess;
+    if (p <= kLuciSolveMax) {
+        const int64_t prod = leftorth ? p * n : m * p, nv = leftorth ? m : n;
+        const size_t lds = (size_t)p * 64 * sizeof(double);
+        if (lds > 64 * 1024) {
+            const hipError_t e = hipFuncSetAttribute((const void *)tci_luci_solve_kernel,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) return e;
+        }
+        hipLaunchKernelGGL(tci_luci_product_kernel, dim3((unsigned)std::min<int64_t>((prod + 255) / 256, 65535)),
+                           dim3(256), 0, st, m, n, p, leftorth, rowperm, colperm, L, U, left, ldl, right, ldr);
+        if (leftorth)
+            hipLaunchKernelGGL(tci_luci_solve_kernel, dim3((unsigned)((nv + 63) / 64)), dim3(64), lds, st, nv, m, (int)p,
+                               1, rowperm, L, L, m, left, ldl);
+        else
+            hipLaunchKernelGGL(tci_luci_solve_kernel, dim3((unsigned)((nv + 63) / 64)), dim3(64), lds, st, nv, m, (int)p,
+                               0, colperm, U, UT, p, right, ldr);
+        return hipGetLastError();
+    }
     int64_t blocks = (tot + 255) / 256;
     if (blocks > 65535) blocks = 65535;
     hipLaunchKernelGGL(tci_luci_kernel, dim3((unsigned)blocks), dim3(256), 0, st, m, n, p, leftorth, rowperm, colperm,
@@ -1296,15 +1432,12 @@ hipError_t launch_rrlu_tile(tci_lu_job *jobs, const int32_t *idx, int64_t count,
     return hipGetLastError();
 }
 
-hipError_t launch_lu_unpack(const double *A, int64_t m, int64_t n, int64_t p, int leftorth,
-                            double *L, int64_t ldl, double *U, int64_t ldu, hipStream_t st)
+hipError_t launch_lu_unpack(const tci_lu_job *job, int64_t most, double *L, double *U, double *diag, double *UT,
+                            hipStream_t st)
 {
-    int64_t tot = m * p + p * n;
-    if (tot == 0) return hipSuccess;
-    int64_t blocks = (tot + 255) / 256;
-    if (blocks > 65535) blocks = 65535;
-    hipLaunchKernelGGL(tci_lu_unpack_kernel, dim3((unsigned)blocks), dim3(256), 0, st, A, m, n, p,
-                       leftorth, L, ldl, U, ldu);
+    if (most <= 0) return hipSuccess;
+    hipLaunchKernelGGL(tci_lu_unpack_kernel, dim3((unsigned)std::min<int64_t>((most + 255) / 256, 4096)), dim3(256), 0,
+                       st, job, L, U, diag, UT);
     return hipGetLastError();
 }
 
