@@ -51,6 +51,15 @@ ENG_INLINE double eng_as_f64(int64_t i)
     return x;
 }
 
+// doubles known to lie in LDS or in memory: accesses through a plain pointer may
+// be to either, and every wait for one kind then waits for the other too
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(3))) double EngLds;
+typedef __attribute__((address_space(1))) double EngGlobal;
+#else
+typedef double EngLds, EngGlobal;
+#endif
+
 ENG_INLINE uint32_t eng_umin(uint32_t a, uint32_t b) { return a < b ? a : b; }
 
 // Base.max on Float64: NaN-propagating

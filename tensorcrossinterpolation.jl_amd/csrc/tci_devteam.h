@@ -35,6 +35,8 @@ __device__ __forceinline__ double readlane_f64(double v, int l)
                             __builtin_amdgcn_readlane(__double2loint(v), l));
 }
 // DPP controls: quad_perm [1,0,3,2] and [2,3,0,1], half-row mirror, row mirror
+// lane 15 of a row to the next row, lane 31 to the upper half
+constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
 
 // WPE (waves per SIMD the kernel is compiled for) is part of the type so
@@ -46,24 +48,56 @@ struct DevTeam {
     static constexpr int RA = TileShape<NT>::RA, CB = TileShape<NT>::CB;
     static constexpr int TMR = WS * RA;   // rows of one wave's staged column
     // LDS of the register-tile rrLU (one set per kernel instantiation)
-    __device__ static double *lds_a() { __shared__ double b[NW]; return b; }
-    __device__ static uint32_t *lds_b() { __shared__ uint32_t b[NW]; return b; }
-    __device__ static double *lds_x() { __shared__ double b[NW * TMR]; return b; }
-    __device__ static double *lds_y() { __shared__ double b[NW * CB]; return b; }
+    __device__ static double *lds_a() { __shared__ double b[2 * NW]; return b; }
+    __device__ static uint32_t *lds_b() { __shared__ uint32_t b[2 * NW]; return b; }
+    __device__ static double *lds_x() { __shared__ double b[2 * NW * TMR]; return b; }
+    __device__ static double *lds_y() { __shared__ double b[NW * 2 * CB]; return b; }
     __device__ double &tA(int w) const { return lds_a()[w]; }
     __device__ uint32_t &tB(int w) const { return lds_b()[w]; }
     __device__ double &tX(int w, int r) const { return lds_x()[w * TMR + r]; }
-    __device__ double &tY(int w, int j) const { return lds_y()[w * CB + j]; }
+    __device__ double &tY(int w, int j) const { return lds_y()[2 * (w * CB + j)]; }
 
-    // wave-uniform max of non-NaN doubles
+    // wave-uniform max of non-NaN doubles (by the instruction itself: fmax of values
+    // moved between lanes costs another one to quieten them; the last two steps
+    // leave the maximum in lane 63)
+    __device__ static double max_raw(double a, double b)
+    {
+        double r;
+        asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+        return r;
+    }
     __device__ double wave_max(double v) const
     {
-        v = fmax(v, dpp_f64<kDppXor1>(v));
-        v = fmax(v, dpp_f64<kDppXor2>(v));
-        v = fmax(v, dpp_f64<kDppHalfMirror>(v));
-        v = fmax(v, dpp_f64<kDppMirror>(v));
-        return fmax(fmax(readlane_f64(v, 0), readlane_f64(v, 16)),
-                    fmax(readlane_f64(v, 32), readlane_f64(v, 48)));
+        v = max_raw(v, dpp_f64<kDppXor1>(v));
+        v = max_raw(v, dpp_f64<kDppXor2>(v));
+        v = max_raw(v, dpp_f64<kDppHalfMirror>(v));
+        v = max_raw(v, dpp_f64<kDppMirror>(v));
+        v = max_raw(v, dpp_f64<kDppBcast15>(v));
+        v = max_raw(v, dpp_f64<kDppBcast31>(v));
+        return readlane_f64(v, 63);
+    }
+    // Of the NW slots from tA(at), tB(at), the smallest key among those whose value's
+    // square is the largest one's (UINT32_MAX when every value is below 0), and the
+    // slot that holds it, counted from at.  Lane l looks at slot l mod NW.
+    __device__ int best_slot(int at, uint32_t &K) const
+    {
+        const int q = at + (lane() & (NW - 1));
+        const double v = tA(q);
+        const uint32_t key = tB(q);
+        double g = v;
+        if constexpr (NW > 1) g = max_raw(g, dpp_f64<kDppXor1>(g));
+        if constexpr (NW > 2) g = max_raw(g, dpp_f64<kDppXor2>(g));
+        if constexpr (NW > 4) g = max_raw(g, dpp_f64<kDppHalfMirror>(g));
+        if constexpr (NW > 8) g = max_raw(g, dpp_f64<kDppMirror>(g));
+        uint32_t k = v >= 0.0 && v * v == g * g ? key : 0xffffffffu;
+        if constexpr (NW > 1) k = min(k, dpp_u32<kDppXor1>(k));
+        if constexpr (NW > 2) k = min(k, dpp_u32<kDppXor2>(k));
+        if constexpr (NW > 4) k = min(k, dpp_u32<kDppHalfMirror>(k));
+        if constexpr (NW > 8) k = min(k, dpp_u32<kDppMirror>(k));
+        K = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);
+        // (a key names one entry of the matrix, so one slot holds it)
+        const unsigned long long b = __ballot(key == K);
+        return b ? (int)__builtin_ctzll(b) & (NW - 1) : 0;
     }
     __device__ uint32_t wave_min(uint32_t v) const
     {

@@ -289,6 +289,16 @@ struct Engine {
     using TileR = TileLU<Team, 1, TCB>;
     using TileC = TileLU<Team, TRA, TCBN>;
     using TileRC = TileLU<Team, 1, TCBN>;
+    // beyond the team's tile, up to 256×256: narrow matrices, and the others by
+    // rows per lane, what the registers do not hold in LDS or memory.  On 512
+    // threads, whose registers hold most of such a matrix; not for the quantics
+    // Gaussians, whose two rows per index seldom reach it, as the kernel body pays
+    // for the call (48 solves of 30 sites 30.3 ms with it, 28.3 without)
+    static constexpr bool EXT = Team::NT == 512 && FK != TCI_F_QUANTICS_GAUSS_COS;
+    using TileN = TileLU<Team, 4, 4, true>;
+    using Tile2 = TileLU<Team, 2, 32, true>;
+    using Tile3 = TileLU<Team, 3, 24, true>;
+    using Tile4 = TileLU<Team, 4, 18, true>;
     Team &tm;
     const SolveDesc &D;
     EngShared &S;
@@ -806,41 +816,64 @@ struct Engine {
                                  double abstol, bool leftorth, double *perr, double *st, double *Lorig)
     {
         T R;
-        R.setup(tm, m, n);
-        R.load(tm, A, m);
+        R.setup(tm, tm.uniform(m), tm.uniform(n));
+        R.load_known(tm, A, m, A == tm.lpi);
         return R.factor(tm, maxrank, reltol, abstol, leftorth, pvals, perr, st, Lorig, rperm, cperm);
     }
 
-    // rrlu!(A) on the m×n matrix A (lda = m).  With need_left, A's first p
-    // columns hold the factor L in position order afterwards (used by
-    // colstimespivotinv); otherwise only the permutations, pivots and error
-    // are produced.  Small matrices are factored in registers.
-    // (not inlined: one copy of the register tile code per kernel)
-    ENG_NOINLINE int rrlu(double *A, int m, int n, int64_t maxrank, double reltol, double abstol,
-                          bool leftorth, double *perr, bool need_left = false,
-                          double *lscratch = nullptr)
+    // Room of an extended tile in LDS: its staging in the rrLU staging vectors,
+    // else in the Pi area (free from lfree), and its columns in what those leave
+    template <class T>
+    ENG_INLINE bool ext_room(int64_t lfree, double *&stage, double *&r1, int64_t &n1, double *&r2, int64_t &n2) const
     {
-        double st[4];
-        const uint64_t t0 = tm.clock();
-        int p;
-        if (Team::RA > 0 && Tile::fits(m, n)) {
-            // L recorded by original row in lscratch, then permuted into A
-            double *Lorig = need_left ? lscratch : nullptr;
-            if (TileRC::fits(m, n)) p = tile_factor<TileRC>(A, m, n, maxrank, reltol, abstol, leftorth, perr, st, Lorig);
-            else if (TileR::fits(m, n)) p = tile_factor<TileR>(A, m, n, maxrank, reltol, abstol, leftorth, perr, st, Lorig);
-            else if (TileC::fits(m, n)) p = tile_factor<TileC>(A, m, n, maxrank, reltol, abstol, leftorth, perr, st, Lorig);
-            else p = tile_factor<Tile>(A, m, n, maxrank, reltol, abstol, leftorth, perr, st, Lorig);
-            if (need_left && p > 0) {
-                tm.sync();
-                for (int t = tm.wave(); t < p; t += tm.nwaves())
-                    for (int pos = t + 1 + tm.lane(); pos < m; pos += tm.wsize())
-                        A[pos + (int64_t)m * t] = Lorig[rperm[pos] + (int64_t)m * t];
-            }
-            tm.sync();
-        } else {
-            p = rrlu_team(tm, A, m, n, maxrank, reltol, abstol, leftorth, rperm, cperm,
-                          pvals, perr, st);
+        const int64_t sv = tm.stage_lds ? 2 * (int64_t)D.mrcap : 0;
+        r2 = tm.lpi + lfree;
+        n2 = tm.lpi && tm.lpi_cap > lfree ? tm.lpi_cap - lfree : 0;
+        r1 = tm.xs;
+        n1 = sv;
+        if (sv >= T::STAGE) {
+            stage = tm.xs;
+            r1 += T::STAGE;
+            n1 -= T::STAGE;
+            return true;
         }
+        if (n2 < T::STAGE) return false;
+        stage = r2;
+        r2 += T::STAGE;
+        n2 -= T::STAGE;
+        return true;
+    }
+
+    // the factorization with an extended tile; false when LDS does not hold its staging
+    template <class T>
+    ENG_INLINE bool ext_tile(int64_t lfree, double *A, int m, int n, int64_t maxrank, double reltol, double abstol,
+                             bool leftorth, double *perr, double *st, double *Lorig, int &p)
+    {
+        double *stage, *r1, *r2;
+        int64_t n1, n2;
+        if (!ext_room<T>(lfree, stage, r1, n1, r2, n2)) return false;
+        const bool inlds = A == tm.lpi;
+        T R;
+        R.setup(tm, tm.uniform(m), tm.uniform(n));
+        R.place(tm, stage, r1, n1, r2, n2, A, inlds);
+        tm.sync();   // (the staging vectors were read by others)
+        R.load_known(tm, A, m, inlds);
+        R.load_extra(tm, A, inlds);
+        p = R.factor(tm, maxrank, reltol, abstol, leftorth, pvals, perr, st, Lorig, rperm, cperm);
+        return true;
+    }
+
+    // counters of a factorization, and L recorded by original row in Lorig permuted
+    // into A's first p columns; ends with a barrier
+    ENG_INLINE void rrlu_done(uint64_t t0, double *A, int m, int n, int p, const double *st, const double *Lorig)
+    {
+        if (Lorig && p > 0) {
+            tm.sync();
+            for (int t = tm.wave(); t < p; t += tm.nwaves())
+                for (int pos = t + 1 + tm.lane(); pos < m; pos += tm.wsize())
+                    A[pos + (int64_t)m * t] = Lorig[rperm[pos] + (int64_t)m * t];
+        }
+        tm.sync();
         if (tm.tid() == 0) {
             S.tph[PH_RRLU] += tm.clock() - t0;
             S.ws[1] += 8.0 * st[0];
@@ -849,6 +882,67 @@ struct Engine {
             S.ws[3] += 2.0 * st[1];
             S.ws[4] += 1.0;
         }
+    }
+
+    static constexpr int kNoRoom = -1000;   // rrlu_ext: LDS does not hold the tile's staging
+
+    // the factorization with an extended tile (as rrlu)
+    ENG_NOINLINE int rrlu_ext(int64_t lfree, double *A, int m, int n, int64_t maxrank, double reltol, double abstol,
+                              bool leftorth, double *perr, double *Lorig)
+    {
+        double st[4];
+        const uint64_t t0 = tm.clock();
+        int p;
+        bool done;
+        if (n <= TileN::NW * 4)
+            done = ext_tile<TileN>(lfree, A, m, n, maxrank, reltol, abstol, leftorth, perr, st, Lorig, p);
+        else if (m <= Tile2::MR)
+            done = ext_tile<Tile2>(lfree, A, m, n, maxrank, reltol, abstol, leftorth, perr, st, Lorig, p);
+        else if (m <= Tile3::MR)
+            done = ext_tile<Tile3>(lfree, A, m, n, maxrank, reltol, abstol, leftorth, perr, st, Lorig, p);
+        else done = ext_tile<Tile4>(lfree, A, m, n, maxrank, reltol, abstol, leftorth, perr, st, Lorig, p);
+        if (!done) return kNoRoom;
+        rrlu_done(t0, A, m, n, p, st, Lorig);
+        return p;
+    }
+
+    // the factorization in the team's tile or streamed (as rrlu)
+    ENG_NOINLINE int rrlu_tile(double *A, int m, int n, int64_t maxrank, double reltol, double abstol,
+                               bool leftorth, double *perr, double *Lorig)
+    {
+        double st[4];
+        const uint64_t t0 = tm.clock();
+        int p;
+        if (Team::RA > 0 && Tile::fits(m, n)) {
+            if (TileRC::fits(m, n)) p = tile_factor<TileRC>(A, m, n, maxrank, reltol, abstol, leftorth, perr, st, Lorig);
+            else if (TileR::fits(m, n)) p = tile_factor<TileR>(A, m, n, maxrank, reltol, abstol, leftorth, perr, st, Lorig);
+            else if (TileC::fits(m, n)) p = tile_factor<TileC>(A, m, n, maxrank, reltol, abstol, leftorth, perr, st, Lorig);
+            else p = tile_factor<Tile>(A, m, n, maxrank, reltol, abstol, leftorth, perr, st, Lorig);
+        } else {
+            p = rrlu_team(tm, A, m, n, maxrank, reltol, abstol, leftorth, rperm, cperm, pvals, perr, st);
+            Lorig = nullptr;   // (L is in A)
+        }
+        rrlu_done(t0, A, m, n, p, st, Lorig);
+        return p;
+    }
+
+    // rrlu!(A) on the m×n matrix A (lda = m).  With need_left, A's first p
+    // columns hold the factor L in position order afterwards (used by
+    // colstimespivotinv); otherwise only the permutations, pivots and error
+    // are produced.  Small matrices are factored in registers.  lfree: first
+    // double of the LDS Pi area beyond A and the permutations (perm_area).
+    // (One copy of the tile code per kernel, the extended tiles apart and marked
+    // unlikely: their registers are all of them, and the values of the kernel
+    // body would be kept in scratch for every solve, not just around their call)
+    ENG_INLINE int rrlu(int64_t lfree, double *A, int m, int n, int64_t maxrank, double reltol, double abstol,
+                        bool leftorth, double *perr, bool need_left = false, double *lscratch = nullptr)
+    {
+        double *Lorig = need_left ? lscratch : nullptr;
+        int p = kNoRoom;
+        if constexpr (EXT)
+            if (__builtin_expect(!Tile::fits(m, n) && m <= 256 && n <= 256, 0))
+                p = rrlu_ext(lfree, A, m, n, maxrank, reltol, abstol, leftorth, perr, Lorig);
+        if (p == kNoRoom) p = rrlu_tile(A, m, n, maxrank, reltol, abstol, leftorth, perr, Lorig);
         return p;
     }
 
@@ -977,9 +1071,9 @@ struct Engine {
             p = eval_rrlu_lorentz(m, b + 1, n, D.maxbonddim, 1e-14, abstol, leftorth, &err);
         } else {
             double *A = pibuf(m, n);
-            perm_area(A == tm.lpi ? (((int64_t)m * n + 1) & ~(int64_t)1) : 0, m, n);
+            const int64_t off = perm_area(A == tm.lpi ? (((int64_t)m * n + 1) & ~(int64_t)1) : 0, m, n);
             eval(rows, b + 1, m, cols, n, A, m, false, true);
-            p = rrlu(A, m, n, D.maxbonddim, 1e-14, abstol, leftorth, &err);
+            p = rrlu(off, A, m, n, D.maxbonddim, 1e-14, abstol, leftorth, &err);
         }
         if (p < 0) return fail(-p);
         if (p > D.setcap) return fail(ST_CAPACITY);
@@ -1144,9 +1238,9 @@ struct Engine {
                 ms = colmove ? nI0 : m;
                 ns = colmove ? n : nJ0;
                 double *A = pibuf(ms, ns);
-                perm_area(A == tm.lpi ? (((int64_t)ms * ns + 1) & ~(int64_t)1) : 0, ms, ns);
+                const int64_t off = perm_area(A == tm.lpi ? (((int64_t)ms * ns + 1) & ~(int64_t)1) : 0, ms, ns);
                 eval_idx(nl, ri, ms, ci, ns, A, ms);
-                p = rrlu(A, ms, ns, maxrank, 1e-14, abstol, leftorth, &e);
+                p = rrlu(off, A, ms, ns, maxrank, 1e-14, abstol, leftorth, &e);
                 if (p < 0) return p;
                 // the swaps of this factorization act on RP/CP's first ms/ns entries
                 for (int i = tm.tid(); i < ms; i += tm.nt()) ta[i] = RP[rperm[i]];
@@ -1842,7 +1936,7 @@ struct Engine {
             int64_t off = perm_area(A == tm.lpi ? (((int64_t)m * nJ + 1) & ~(int64_t)1) : 0, m, nJ);
             eval(rows, b + 1, m, cols, nJ, A, m, false, true);
             double err;
-            int p = rrlu(A, m, nJ, D.maxbonddim, 1e-14, abstol, true, &err, true, Tslot(b));
+            int p = rrlu(off, A, m, nJ, D.maxbonddim, 1e-14, abstol, true, &err, true, Tslot(b));
             if (p < 0) {
                 if (tm.tid() == 0) D.ints[INT_ERRSITE] = b + 1;
                 return fail(-p);

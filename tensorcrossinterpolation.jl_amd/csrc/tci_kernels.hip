@@ -326,7 +326,7 @@ __device__ void tile_job(Team &tm, tci_lu_job &J, int m, int n, double *Lsc, dou
     if (n < mr) mr = n;
     T R;
     R.setup(tm, m, n);
-    R.load(tm, J.A, m);
+    R.load_known(tm, J.A, m, false);
     __syncthreads();   // every load of A done before A is rewritten
     double err, st[2];
     const int p = R.factor(tm, J.maxrank, J.reltol, J.abstol, J.leftorth != 0, pv, &err, st, Lsc,

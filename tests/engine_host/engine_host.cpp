@@ -20,11 +20,12 @@ using namespace tci;
 struct HostTeam {
     // register tile of the one-thread team: one wave of one lane holding up to 160×160
     static constexpr int NT = 1, WS = 1, NW = 1, RA = 160, CB = 160, WPE = 1;
-    double lA[1], lX[160], lY[160];
-    uint32_t lB[1];
-    double &tA(int) { return lA[0]; }
-    uint32_t &tB(int) { return lB[0]; }
-    double &tX(int, int r) { return lX[r]; }
+    double lA[2], lX[2 * 160], lY[160];
+    uint32_t lB[2];
+    int best_slot(int at, uint32_t &K) { K = lA[at] >= 0.0 ? lB[at] : 0xffffffffu; return 0; }
+    double &tA(int w) { return lA[w]; }
+    uint32_t &tB(int w) { return lB[w]; }
+    double &tX(int w, int r) { return lX[160 * w + r]; }
     double &tY(int, int j) { return lY[j]; }
     int tid() const { return 0; }
     static constexpr int nt() { return 1; }
@@ -76,8 +77,8 @@ struct MTShared {
 
 template <int NT_, int RA_, int CB_>
 struct MTTile {
-    double A[NT_ / 64], X[(NT_ / 64) * 64 * RA_], Y[(NT_ / 64) * CB_];
-    uint32_t B[NT_ / 64];
+    double A[2 * NT_ / 64], X[(2 * NT_ / 64) * 64 * RA_], Y[(NT_ / 64) * CB_];
+    uint32_t B[2 * NT_ / 64];
 };
 
 template <int NT_, int RA_, int CB_>
@@ -86,6 +87,20 @@ struct HostTeamMT {
     MTTile<NT_, RA_, CB_> *tile = nullptr;
     double &tA(int w) { return tile->A[w]; }
     uint32_t &tB(int w) { return tile->B[w]; }
+    // of the slots from at, the smallest key of those that reach the largest square
+    int best_slot(int at, uint32_t &K)
+    {
+        double g = -1.0;
+        for (int q = 0; q < NW; ++q) g = tA(at + q) > g ? tA(at + q) : g;
+        K = 0xffffffffu;
+        int w = 0;
+        for (int q = 0; q < NW; ++q)
+            if (tA(at + q) >= 0.0 && tA(at + q) * tA(at + q) == g * g && tB(at + q) < K) {
+                K = tB(at + q);
+                w = q;
+            }
+        return w;
+    }
     double &tX(int w, int r) { return tile->X[w * 64 * RA + r]; }
     double &tY(int w, int j) { return tile->Y[w * CB + j]; }
     int t_tid = 0;
@@ -242,6 +257,63 @@ extern "C" int eh_rrlu_mt(int mode, double *A, int m, int n, int64_t maxrank, do
     for (int j = 0; j < n; ++j) colperm[j] = cp[j];
     *err = eres;
     return pres;
+}
+
+// rrlu! through an extended tile (columns beyond the registers in two areas of
+// n1 and n2 doubles, then in the matrix itself; all of them there when inplace)
+// on 256 host threads.  shape: 0 4×18, 1 3×24, 2 2×32, 3 4×4 doubles a lane.
+template <int RA, int CB>
+static int ext_mt(int64_t n1, int64_t n2, int inplace, double *A, int m, int n, int64_t maxrank, double reltol,
+                  double abstol, int leftorth, int32_t *rowperm, int32_t *colperm, double *Lorig, double *err)
+{
+    constexpr int NT = 256;
+    using Team = HostTeamMT<NT, 2, 32>;
+    using Tile = TileLU<Team, RA, CB, true>;
+    if (!Tile::fits(m, n)) return -100;
+    std::barrier<> bar(NT);
+    std::vector<std::barrier<> *> wb;
+    for (int w = 0; w < NT / 64; ++w) wb.push_back(new std::barrier<>(64));
+    MTShared sh;
+    sh.bar = &bar;
+    sh.wbar = wb;
+    sh.abuf.resize(NT);
+    sh.dbuf.resize(NT);
+    sh.ibuf.resize(NT);
+    sh.ubuf.resize(NT);
+    MTTile<NT, 2, 32> tile;
+    std::vector<double> stage(Tile::STAGE), r1(n1 + 1), r2(n2 + 1);
+    int pres = 0;
+    double eres = 0;
+    auto body = [&](int tid) {
+        Team tm;
+        tm.t_tid = tid;
+        tm.sh = &sh;
+        tm.tile = &tile;
+        Tile R;
+        R.setup(tm, m, n);
+        R.place(tm, stage.data(), r1.data(), n1, r2.data(), n2, A, inplace != 0);
+        R.load(tm, A, m);
+        R.load_extra(tm, A, inplace != 0);
+        tm.sync();
+        double e, st[2];
+        int p = R.factor(tm, maxrank, reltol, abstol, leftorth != 0, nullptr, &e, st, Lorig, rowperm, colperm);
+        tm.sync();
+        if (tid == 0) { pres = p; eres = e; }
+    };
+    std::vector<std::thread> th;
+    for (int t = 0; t < NT; ++t) th.emplace_back(body, t);
+    for (auto &t : th) t.join();
+    for (auto *b : wb) delete b;
+    *err = eres;
+    return pres;
+}
+
+extern "C" int eh_rrlu_ext_mt(int shape, int64_t n1, int64_t n2, int inplace, double *A, int m, int n,
+                              int64_t maxrank, double reltol, double abstol, int leftorth, int32_t *rowperm,
+                              int32_t *colperm, double *Lorig, double *err)
+{
+    const auto f = shape == 0 ? ext_mt<4, 18> : shape == 1 ? ext_mt<3, 24> : shape == 2 ? ext_mt<2, 32> : ext_mt<4, 4>;
+    return f(n1, n2, inplace, A, m, n, maxrank, reltol, abstol, leftorth, rowperm, colperm, Lorig, err);
 }
 
 struct EhSolve {
