@@ -2355,8 +2355,23 @@ tci_status tci_tt_floatingzone_f64(tci_ctx *ctx, const tci_functor *f, int32_t L
     if (!points_in_range(L, localdims, npts, points)) return set_err(TCI_ERR_ARG, "point index out of range");
     HIPCHK(hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
-    const int blocks = (int)(npts < 1024 ? npts : 1024);
-    const int64_t wstride = roff[(size_t)L] + chimax + dmax * chimax + dmax;
+    FzArgs fz;
+    memset(&fz, 0, sizeof fz);
+    fz.L = L;
+    fz.chimax = (int)chimax;
+    fz.dmax = (int)dmax;
+    fz.fkind = f->kind;
+    fz.nft = term_functions(*f, L, (int)dmax);
+    fz.nenv = roff[(size_t)L];
+    fz.npts = npts;
+    fz.nsweeps = nsweeps;
+    fz.earlystoptol = earlystoptol;
+    const size_t area = fz_area_bytes(fz);
+    fz.wstride = (int64_t)((area + 7) / 8);
+    const int64_t most = area > kFzLds ? 1024 : 2048;   // eight workgroups per CU
+    const int blocks = (int)(npts < most ? npts : most);
+    int64_t slice = 0;
+    for (int b = 1; b < L; ++b) slice += linkdims[b] * linkdims[b + 1];
     size_t need = 0;
     auto a = [&](size_t bytes) { size_t at = need; need = lay_align(need + (bytes ? bytes : 1)); return at; };
     const size_t o_c = a(sizeof(double) * (size_t)tot);
@@ -2367,8 +2382,8 @@ tci_status tci_tt_floatingzone_f64(tci_ctx *ctx, const tci_functor *f, int32_t L
     const size_t o_ipar = a(sizeof(int32_t) * (size_t)f->niparams);
     const size_t o_pts = a((size_t)(npts * L));
     const size_t o_err = a(sizeof(double) * (size_t)npts);
-    const size_t o_w = a(sizeof(double) * (size_t)(wstride * blocks));
-    const size_t o_dig = a((size_t)(dmax * L * blocks));
+    const size_t o_w = a(area > kFzLds ? sizeof(double) * (size_t)(fz.wstride * blocks) : 0);
+    const size_t o_ft = a(sizeof(double) * (size_t)fz.nft * (size_t)(L * dmax));
     uint8_t *d = nullptr;
     HIPCHK(hipMallocAsync((void **)&d, need, st));
     hipError_t e = hipMemcpyAsync(d + o_c, cores, sizeof(double) * (size_t)tot, hipMemcpyHostToDevice, st);
@@ -2380,12 +2395,16 @@ tci_status tci_tt_floatingzone_f64(tci_ctx *ctx, const tci_functor *f, int32_t L
     if (e == hipSuccess && f->niparams)
         e = hipMemcpyAsync(d + o_ipar, f->iparams, sizeof(int32_t) * f->niparams, hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hipMemcpyAsync(d + o_pts, points, (size_t)(npts * L), hipMemcpyHostToDevice, st);
-    if (e == hipSuccess)
-        e = launch_floatingzone(L, (const int64_t *)(d + o_d), (const int64_t *)(d + o_o), (const double *)(d + o_c),
-                                (const int64_t *)(d + o_r), (int)chimax, (int)dmax, f->kind,
-                                (const double *)(d + o_par), (const int32_t *)(d + o_ipar), d + o_pts,
-                                (double *)(d + o_err), npts, nsweeps, earlystoptol, (double *)(d + o_w), wstride,
-                                d + o_dig, blocks, st);
+    fz.dims3 = (const int64_t *)(d + o_d);
+    fz.coff = (const int64_t *)(d + o_o);
+    fz.roff = (const int64_t *)(d + o_r);
+    fz.cores = (const double *)(d + o_c);
+    fz.params = (const double *)(d + o_par);
+    fz.iparams = (const int32_t *)(d + o_ipar);
+    fz.pts = d + o_pts;
+    fz.errs = (double *)(d + o_err);
+    fz.work = (double *)(d + o_w);
+    if (e == hipSuccess) e = launch_floatingzone(fz, slice, blocks, (double *)(d + o_ft), st);
     if (e == hipSuccess) e = hipMemcpyAsync(points, d + o_pts, (size_t)(npts * L), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipMemcpyAsync(errors, d + o_err, sizeof(double) * (size_t)npts, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);

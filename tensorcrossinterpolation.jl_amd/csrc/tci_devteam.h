@@ -34,9 +34,9 @@ __device__ __forceinline__ double readlane_f64(double v, int l)
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
                             __builtin_amdgcn_readlane(__double2loint(v), l));
 }
-// DPP controls: quad_perm [1,0,3,2] and [2,3,0,1], half-row mirror, row mirror
-// lane 15 of a row to the next row, lane 31 to the upper half
+// DPP controls: lane 15 of a row to the next row, lane 31 to the upper half
 constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;
+// quad_perm [1,0,3,2] and [2,3,0,1], half-row mirror, row mirror
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
 
 // WPE (waves per SIMD the kernel is compiled for) is part of the type so
@@ -57,23 +57,15 @@ struct DevTeam {
     __device__ double &tX(int w, int r) const { return lds_x()[w * TMR + r]; }
     __device__ double &tY(int w, int j) const { return lds_y()[2 * (w * CB + j)]; }
 
-    // wave-uniform max of non-NaN doubles (by the instruction itself: fmax of values
-    // moved between lanes costs another one to quieten them; the last two steps
-    // leave the maximum in lane 63)
-    __device__ static double max_raw(double a, double b)
-    {
-        double r;
-        asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-        return r;
-    }
+    // wave-uniform max of non-NaN doubles (the last two steps leave it in lane 63)
     __device__ double wave_max(double v) const
     {
-        v = max_raw(v, dpp_f64<kDppXor1>(v));
-        v = max_raw(v, dpp_f64<kDppXor2>(v));
-        v = max_raw(v, dpp_f64<kDppHalfMirror>(v));
-        v = max_raw(v, dpp_f64<kDppMirror>(v));
-        v = max_raw(v, dpp_f64<kDppBcast15>(v));
-        v = max_raw(v, dpp_f64<kDppBcast31>(v));
+        v = fmax(v, dpp_f64<kDppXor1>(v));
+        v = fmax(v, dpp_f64<kDppXor2>(v));
+        v = fmax(v, dpp_f64<kDppHalfMirror>(v));
+        v = fmax(v, dpp_f64<kDppMirror>(v));
+        v = fmax(v, dpp_f64<kDppBcast15>(v));
+        v = fmax(v, dpp_f64<kDppBcast31>(v));
         return readlane_f64(v, 63);
     }
     // Of the NW slots from tA(at), tB(at), the smallest key among those whose value's
@@ -85,10 +77,10 @@ struct DevTeam {
         const double v = tA(q);
         const uint32_t key = tB(q);
         double g = v;
-        if constexpr (NW > 1) g = max_raw(g, dpp_f64<kDppXor1>(g));
-        if constexpr (NW > 2) g = max_raw(g, dpp_f64<kDppXor2>(g));
-        if constexpr (NW > 4) g = max_raw(g, dpp_f64<kDppHalfMirror>(g));
-        if constexpr (NW > 8) g = max_raw(g, dpp_f64<kDppMirror>(g));
+        if constexpr (NW > 1) g = fmax(g, dpp_f64<kDppXor1>(g));
+        if constexpr (NW > 2) g = fmax(g, dpp_f64<kDppXor2>(g));
+        if constexpr (NW > 4) g = fmax(g, dpp_f64<kDppHalfMirror>(g));
+        if constexpr (NW > 8) g = fmax(g, dpp_f64<kDppMirror>(g));
         uint32_t k = v >= 0.0 && v * v == g * g ? key : 0xffffffffu;
         if constexpr (NW > 1) k = min(k, dpp_u32<kDppXor1>(k));
         if constexpr (NW > 2) k = min(k, dpp_u32<kDppXor2>(k));

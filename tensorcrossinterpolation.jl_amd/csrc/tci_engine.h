@@ -272,6 +272,19 @@ ENG int rrlu_team(Team &tm, double *A, int m, int n, int64_t maxrank, double rel
 }
 
 
+// term of site t at index v in the k-th of a functor's nft sums over sites, by the
+// functor's own operations (weighted Lorentzian: one sum; Gaussian sum: one each)
+ENG inline double term_value(int kind, const double *p, int nft, int L, int k, int t, int v)
+{
+    if (kind == TCI_F_LORENTZ_WEIGHTED) {
+        const double u = (double)v / p[0];
+        return p[1 + t] * (u * u);
+    }
+    const double xi = (double)(v - 1) / (p[1] - 1.0);
+    const double u = xi - p[2 + 2 * nft + k * L + t];
+    return u * u;
+}
+
 // phases timed by the engine (ticks of tm.clock(), accumulated by thread 0)
 enum { PH_EVAL = 0, PH_RRLU = 1, PH_SETS = 2, PH_FILL = 3, PH_GSEARCH = 4, PH_SWEEP1 = 5, PH_TOTAL = 6,
        PH_SOLVE = 7 };
@@ -350,17 +363,7 @@ struct Engine {
         const double *p = D.params;
         const int ds = D.dmax, per = L * ds;
         for (int q = tm.tid(); q < D.nftab * per; q += tm.nt()) {
-            const int k = q / per, t = (q - k * per) / ds, v = q % ds + 1;
-            double x = 0.0;
-            if (kind() == TCI_F_LORENTZ_WEIGHTED) {
-                const double u = (double)v / p[0];
-                x = p[1 + t] * (u * u);
-            } else {
-                const double xi = (double)(v - 1) / (p[1] - 1.0);
-                const double u = xi - p[2 + 2 * D.nftab + k * L + t];
-                x = u * u;
-            }
-            D.ftab[q] = x;
+            D.ftab[q] = term_value(kind(), p, D.nftab, L, q / per, q % per / ds, q % ds + 1);
         }
         tm.sync();
     }

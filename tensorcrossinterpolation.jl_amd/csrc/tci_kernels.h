@@ -170,11 +170,32 @@ hipError_t launch_tt_finish(const double *V, int stride, const uint8_t *pts, int
 // _floatingzone from each of npts points (in/out, npts×L digits), one
 // workgroup per point; work: wstride doubles per workgroup, digits: dmax·L
 // bytes per workgroup; roff: L+1 offsets of the right environments
-hipError_t launch_floatingzone(int L, const int64_t *dims3, const int64_t *coff, const double *cores,
-                               const int64_t *roff, int chimax, int dmax, int fkind, const double *params,
-                               const int32_t *iparams, uint8_t *pts, double *errs, int64_t npts, int64_t nsweeps,
-                               double earlystoptol, double *work, int64_t wstride, uint8_t *digits, int blocks,
-                               hipStream_t st);
+// the floating-zone search: points and errors in place, the train as dims3 (three
+// per site), its cores' offsets coff, the environments' offsets roff
+struct FzArgs {
+    int L, chimax, dmax, fkind;
+    int nft;              // per-site term functions of f (0: f evaluated as a whole)
+    int nslice;           // doubles of the slices kept in LDS (0: none)
+    const int64_t *dims3, *coff, *roff;
+    const double *cores, *params, *ftab;
+    const int32_t *iparams;
+    uint8_t *pts;
+    double *errs;
+    int64_t npts, nsweeps;
+    double earlystoptol;
+    double *work;         // per workgroup wstride doubles, when LDS does not hold them
+    int64_t wstride, nenv;
+};
+// LDS of the search: at most kFzLds, with the slices at most kFzSliceLds
+constexpr size_t kFzLds = 60 * 1024, kFzSliceLds = 19 * 1024;
+// bytes of a workgroup's work area without the slices
+inline size_t fz_area_bytes(const FzArgs &a)
+{
+    const size_t dbl = (size_t)a.nenv + 2 * (size_t)a.dmax * a.chimax + (size_t)a.dmax + (size_t)a.nft * (a.dmax + a.L);
+    return sizeof(double) * dbl + (a.nft ? 0 : (((size_t)a.dmax * a.L + 7) & ~(size_t)7));
+}
+// slice: doubles of all T_b[:, x_b, :] beyond the first site
+hipError_t launch_floatingzone(FzArgs a, int64_t slice, int blocks, double *ftab, hipStream_t st);
 hipError_t launch_eval(int kind, const double *params, const int32_t *iparams, int L,
                        const uint8_t *rows, int64_t nrow, int rstride, int nl, const uint8_t *cols,
                        int64_t ncol, int cstride, double *out, double *blockmax, hipStream_t st);

@@ -1150,6 +1150,68 @@ hipError_t launch_tt_finish(const double *V, int stride, const uint8_t *pts, int
     return hipGetLastError();
 }
 
+// the table of a functor's per-site terms (term_value), for f along a site
+__global__ __launch_bounds__(256) void tci_terms_kernel(int kind, const double *__restrict__ params, int nft, int L,
+                                                        int dmax, double *__restrict__ ftab)
+{
+    const int q = blockIdx.x * 256 + threadIdx.x;
+    if (q < nft * L * dmax)
+        ftab[q] = term_value(kind, params, nft, L, q / (L * dmax), q / dmax % L, q % dmax + 1);
+}
+
+// f at the current point with site p at s (0-based): per-site terms summed in the
+// functor's order, cur those of the current point, own those of (p, s); or the
+// functor itself on row, the point's digits
+template <bool TERMS>
+__device__ __forceinline__ double fz_value(const FzArgs &a, const uint8_t *piv, const double *cur, const double *own,
+                                           uint8_t *row, int p, int s)
+{
+    const int L = a.L;
+    if constexpr (!TERMS) {
+        for (int t = 0; t < L; ++t) row[t] = t == p ? (uint8_t)(s + 1) : piv[t];
+        tci_point x;
+        x.a = row;
+        x.b = row;
+        x.na = L;
+        x.L = L;
+        return tci_functor_eval(a.fkind, a.params, a.iparams, &x);
+    }
+    double f = 0.0;
+    for (int k = 0; k < a.nft; ++k) {
+        const double *c = cur + k * L;
+        double u = 0.0;
+        const double mine = own[k * a.dmax + s];
+#pragma unroll 4
+        for (int t = 0; t < L; ++t) u = u + (t == p ? mine : c[t]);
+        if (a.fkind == TCI_F_LORENTZ_WEIGHTED) return 1.0 / (1.0 + u);
+        const double w = a.params[2 + a.nft + k];
+        f = f + a.params[2 + k] * tci_exp(-u / (2.0 * (w * w)));
+    }
+    return f;
+}
+
+// Σ_j x[j]·T[st·j] in ascending j from 0.0, the loads of eight terms in flight
+// (the last ones clamped and not added)
+__device__ __forceinline__ double fz_dot(const double *x, const double *T, int64_t st, int n)
+{
+    double acc = 0.0;
+    for (int j0 = 0; j0 < n; j0 += 8) {
+        double v[8], y[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int j = j0 + u < n ? j0 + u : n - 1;
+            v[u] = T[st * j];
+            y[u] = x[j];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const double t = y[u] * v[u], sum = acc + t;
+            acc = j0 + u < n ? sum : acc;
+        }
+    }
+    return acc;
+}
+
 // _floatingzone (globalsearch.jl:43-95) from each start point: one
 // workgroup per point (grid-stride).  Per sweep, the right environments
 // R_b = T_b[:, x_b, :]·R_{b+1} (R_L = [1], each entry summed in ascending
@@ -1161,133 +1223,161 @@ hipError_t launch_tt_finish(const double *V, int stride, const uint8_t *pts, int
 // error takes the NaN-propagating max.  A sweep that leaves the error
 // unchanged, or lifts it above earlystoptol, ends the search; so does a
 // NaN error (with which the reference would sweep without end).
-// Work area per workgroup (wstride doubles): renv (Σ_{b=1..L} χ_b, at
-// roff[b-1]) | l (chimax) | w (dmax·chimax) | err (dmax); digit rows
-// (dmax·L bytes per workgroup) hold the candidate points.
-__global__ __launch_bounds__(256) void tci_floatingzone_kernel(
-    int L, const int64_t *__restrict__ dims3, const int64_t *__restrict__ coff, const double *__restrict__ cores,
-    const int64_t *__restrict__ roff, int chimax, int dmax, int fkind, const double *__restrict__ params,
-    const int32_t *__restrict__ iparams, uint8_t *__restrict__ pts, double *__restrict__ errs, int64_t npts,
-    int64_t nsweeps, double earlystoptol, double *__restrict__ work, int64_t wstride, uint8_t *__restrict__ digits)
+// Bound: the latency of a site's steps, which follow each other.  So the work
+// area (renv | w, two of them | f and the terms along the site | the current
+// point's terms | the slices T_b[:, x_b, :] where there is room | digit rows) lies
+// in LDS, f is evaluated by the far end of the workgroup while w is formed, from
+// terms that only differ in site p, and l is a row of the last w: two barriers a
+// site.  With all of it in memory, every f from scratch and one thread looking for
+// the maximum, 2000 starts of 20 sites, d 16, took 7.4 ms; 2.6 so, most of
+// it the few starts that need 20 sweeps and more (0.11 ms each).
+// LDS = false: the same on a work area in memory, for trains that LDS does not hold.
+// TERMS: f by its terms, apart from the functors' own evaluation, whose registers
+// would leave five waves a SIMD of the eight.
+template <bool LDS, bool TERMS>
+__global__ __launch_bounds__(256, TERMS ? 8 : 1) void tci_floatingzone_kernel(FzArgs a)
 {
     __shared__ uint8_t piv[256];
     __shared__ double s_maxerr;
-    __shared__ int s_best, s_stop;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    double *renv = work + (int64_t)blockIdx.x * wstride;
-    double *lv = renv + roff[L];
-    double *w = lv + chimax;
-    double *err = w + (int64_t)dmax * chimax;
-    uint8_t *rows = digits + (int64_t)blockIdx.x * dmax * L;
-    for (int64_t q = blockIdx.x; q < npts; q += gridDim.x) {
-        for (int t = tid; t < L; t += nt) piv[t] = pts[q * L + t];
+    __shared__ int s_best;
+    extern __shared__ double dyn[];
+    DevTeam<256> tm;   // (its wave operations)
+    const int tid = threadIdx.x, nt = 256, L = a.L;
+    double *base;
+    if constexpr (LDS) base = dyn;
+    else base = a.work + (int64_t)blockIdx.x * a.wstride;
+    double *renv = base;
+    double *w0 = renv + a.roff[L];
+    const int64_t wsz = (int64_t)a.dmax * a.chimax;
+    double *fv = w0 + 2 * wsz;
+    double *own = fv + a.dmax;
+    double *cur = own + a.nft * a.dmax;
+    double *sl = cur + a.nft * L;
+    uint8_t *rows = (uint8_t *)(sl + (LDS ? a.nslice : 0));
+    for (int64_t q = blockIdx.x; q < a.npts; q += gridDim.x) {
+        for (int t = tid; t < L; t += nt) piv[t] = a.pts[q * L + t];
         __syncthreads();
         for (int64_t sweep = 0;; ++sweep) {
+            for (int i = tid; i < a.nft * L; i += nt) cur[i] = a.ftab[(int64_t)i * a.dmax + piv[i % L] - 1];
+            if (LDS && a.nslice) {
+                double *to = sl;
+                for (int b = 1; b < L; ++b) {
+                    const int d0 = (int)a.dims3[3 * b], d = (int)a.dims3[3 * b + 1], n = d0 * (int)a.dims3[3 * b + 2];
+                    const double *Tc = a.cores + a.coff[b] + d0 * (int64_t)(piv[b] - 1);
+                    for (int o = tid; o < n; o += nt) to[o] = Tc[o % d0 + (int64_t)d0 * d * (o / d0)];
+                    to += n;
+                }
+            }
             // right environments of the current point
-            if (tid == 0) renv[roff[L - 1]] = 1.0;   // R_L
+            if (tid == 0) {
+                renv[a.roff[L - 1]] = 1.0;   // R_L
+                w0[wsz] = 1.0;               // l before the first site
+            }
             __syncthreads();
+            const double *from = sl + a.nslice;
             for (int b = L - 1; b >= 1; --b) {
-                const int64_t d0 = dims3[3 * b], d = dims3[3 * b + 1], d2 = dims3[3 * b + 2];
-                const double *Tc = cores + coff[b] + d0 * (int64_t)(piv[b] - 1);
-                const double *Rn = renv + roff[b];
-                double *Rb = renv + roff[b - 1];
-                for (int64_t j = tid; j < d0; j += nt) {
-                    double acc = 0.0;
-                    for (int64_t k = 0; k < d2; ++k) acc = acc + Tc[j + d0 * d * k] * Rn[k];
-                    Rb[j] = acc;
+                const int d0 = (int)a.dims3[3 * b], d = (int)a.dims3[3 * b + 1], d2 = (int)a.dims3[3 * b + 2];
+                const double *Rn = renv + a.roff[b];
+                double *Rb = renv + a.roff[b - 1];
+                if (LDS && a.nslice) {
+                    from -= d0 * d2;
+                    for (int j = tid; j < d0; j += nt) Rb[j] = fz_dot(Rn, from + j, d0, d2);
+                } else {
+                    const double *Tc = a.cores + a.coff[b] + d0 * (int64_t)(piv[b] - 1);
+                    for (int j = tid; j < d0; j += nt) Rb[j] = fz_dot(Rn, Tc + j, (int64_t)d0 * d, d2);
                 }
                 __syncthreads();
             }
             if (sweep == 0) {
                 // the start point's error: TT(x) = T_1[1, x_1, :]·R_2
                 if (tid == 0) {
-                    const int64_t d = dims3[1], d2 = dims3[2];
-                    const double *Tc = cores + coff[0] + (int64_t)(piv[0] - 1);
-                    const double *Rn = renv + roff[0];
+                    const int64_t d = a.dims3[1], d2 = a.dims3[2];
+                    const double *Tc = a.cores + a.coff[0] + (int64_t)(piv[0] - 1);
+                    const double *Rn = renv + a.roff[0];
                     double acc = 0.0;
                     for (int64_t k = 0; k < d2; ++k) acc = acc + (0.0 + 1.0 * Tc[d * k]) * Rn[k];
-                    tci_point x;
-                    x.a = piv;
-                    x.b = piv;
-                    x.na = L;
-                    x.L = L;
-                    s_maxerr = fabs(tci_functor_eval(fkind, params, iparams, &x) - acc);
+                    const int x0 = piv[0] - 1;
+                    for (int k = 0; k < a.nft; ++k) own[k * a.dmax + x0] = cur[k * L];
+                    s_maxerr = fabs(fz_value<TERMS>(a, piv, cur, own, rows, 0, x0) - acc);
                 }
                 __syncthreads();
             }
             const double prev = s_maxerr;
-            if (tid == 0) lv[0] = 1.0;
-            __syncthreads();
+            const double *lv = w0 + wsz;
             for (int p = 0; p < L; ++p) {
-                const int64_t d0 = dims3[3 * p], d = dims3[3 * p + 1], d2 = dims3[3 * p + 2];
-                const double *T = cores + coff[p];
-                const double *Rn = renv + roff[p];   // R_{p+1}
-                for (int64_t o = tid; o < d * d2; o += nt) {
-                    const int64_t s = o / d2, k = o - s * d2;
-                    const double *Tc = T + d0 * (s + d * k);
-                    double acc = 0.0;
-                    for (int64_t j = 0; j < d0; ++j) acc = acc + lv[j] * Tc[j];
-                    w[s * chimax + k] = acc;
+                const int d0 = (int)a.dims3[3 * p], d = (int)a.dims3[3 * p + 1], d2 = (int)a.dims3[3 * p + 2];
+                const double *T = a.cores + a.coff[p];
+                const double *Rn = renv + a.roff[p];   // R_{p+1}
+                double *w = w0 + (p & 1) * wsz;
+                for (int s = nt - 1 - tid; s < d; s += nt) {
+                    for (int k = 0; k < a.nft; ++k)
+                        own[k * a.dmax + s] = a.ftab[((int64_t)k * L + p) * a.dmax + s];
+                    fv[s] = fz_value<TERMS>(a, piv, cur, own, rows + (int64_t)s * L, p, s);
                 }
-                for (int64_t o = tid; o < d * L; o += nt) {
-                    const int64_t s = o / L, t = o - s * L;
-                    rows[s * L + t] = t == p ? (uint8_t)(s + 1) : piv[t];
-                }
-                __syncthreads();
-                for (int64_t s = tid; s < d; s += nt) {
-                    double acc = 0.0;
-                    for (int64_t k = 0; k < d2; ++k) acc = acc + w[s * chimax + k] * Rn[k];
-                    tci_point x;
-                    x.a = rows + s * L;
-                    x.b = x.a;
-                    x.na = L;
-                    x.L = L;
-                    err[s] = fabs(tci_functor_eval(fkind, params, iparams, &x) - acc);
+                for (int o = tid; o < d * d2; o += nt) {
+                    const int s = o / d2, k = o - s * d2;
+                    w[(int64_t)s * a.chimax + k] = fz_dot(lv, T + (int64_t)d0 * (s + (int64_t)d * k), 1, d0);
                 }
                 __syncthreads();
-                if (tid == 0) {
-                    int best = 0;
-                    double bv = err[0], mx = err[0];
-                    for (int s = 1; s < (int)d; ++s) {
-                        const double e = err[s];
-                        // isless(bv, e): NaN is above every number, the first NaN stays
-                        if (bv == bv && (e != e || bv < e)) {
-                            best = s;
-                            bv = e;
-                        }
-                        mx = jl_max(mx, e);
+                if (tid < 64) {
+                    // isless order: NaN is above every number, the first of equal ones
+                    double bv = -1.0;
+                    uint32_t bi = 0xffffffffu;
+                    for (int s = tid; s < d; s += 64) {
+                        const double e = fabs(fv[s] - fz_dot(w + (int64_t)s * a.chimax, Rn, 1, d2));
+                        // (by selects: as a branch it was compiled to keep the old bv)
+                        const bool take = (bi == 0xffffffffu) | ((bv == bv) & ((e != e) | (bv < e)));
+                        bi = take ? (uint32_t)s : bi;
+                        bv = take ? e : bv;
                     }
-                    piv[p] = (uint8_t)(best + 1);
-                    s_best = best;
-                    s_maxerr = jl_max(mx, s_maxerr);
+                    const bool nan = bv != bv;
+                    double mx;
+                    uint32_t best;
+                    if (tm.wave_any(nan)) {
+                        best = tm.wave_min(nan ? bi : 0xffffffffu);
+                        mx = tm.wave_bcast_f64(bv, (int)(best & 63u));
+                    } else {
+                        mx = tm.wave_max(bv);
+                        best = tm.wave_min(bv == mx ? bi : 0xffffffffu);
+                    }
+                    for (int k = tid; k < a.nft; k += 64) cur[k * L + p] = own[k * a.dmax + best];
+                    if (tid == 0) {
+                        piv[p] = (uint8_t)(best + 1);
+                        s_best = (int)best;
+                        s_maxerr = jl_max(mx, s_maxerr);
+                    }
                 }
                 __syncthreads();
-                for (int64_t k = tid; k < d2; k += nt) lv[k] = w[s_best * chimax + k];
-                __syncthreads();
+                lv = w + (int64_t)s_best * a.chimax;
             }
-            if (tid == 0) {
-                const double me = s_maxerr;
-                s_stop = me == prev || me > earlystoptol || me != me || sweep + 1 >= nsweeps;
-            }
-            __syncthreads();
-            if (s_stop) break;
+            const double me = s_maxerr;
+            if (me == prev || me > a.earlystoptol || me != me || sweep + 1 >= a.nsweeps) break;
+            __syncthreads();   // (renv, w and cur are rewritten)
         }
-        for (int t = tid; t < L; t += nt) pts[q * L + t] = piv[t];
-        if (tid == 0) errs[q] = s_maxerr;
+        for (int t = tid; t < L; t += nt) a.pts[q * L + t] = piv[t];
+        if (tid == 0) a.errs[q] = s_maxerr;
         __syncthreads();
     }
 }
 
-hipError_t launch_floatingzone(int L, const int64_t *dims3, const int64_t *coff, const double *cores,
-                               const int64_t *roff, int chimax, int dmax, int fkind, const double *params,
-                               const int32_t *iparams, uint8_t *pts, double *errs, int64_t npts, int64_t nsweeps,
-                               double earlystoptol, double *work, int64_t wstride, uint8_t *digits, int blocks,
-                               hipStream_t st)
+hipError_t launch_floatingzone(FzArgs a, int64_t slice, int blocks, double *ftab, hipStream_t st)
 {
-    if (npts <= 0) return hipSuccess;
-    hipLaunchKernelGGL(tci_floatingzone_kernel, dim3((unsigned)blocks), dim3(256), 0, st, L, dims3, coff, cores, roff,
-                       chimax, dmax, fkind, params, iparams, pts, errs, npts, nsweeps, earlystoptol, work, wstride,
-                       digits);
+    if (a.npts <= 0) return hipSuccess;
+    if (a.nft) {
+        const int n = a.nft * a.L * a.dmax;
+        hipLaunchKernelGGL(tci_terms_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a.fkind, a.params,
+                           a.nft, a.L, a.dmax, ftab);
+        a.ftab = ftab;
+    }
+    // the slices where eight workgroups still share a CU (with less, the next
+    // points' loads no longer hide behind each other)
+    const size_t area = fz_area_bytes(a);
+    a.nslice = area + sizeof(double) * (size_t)slice <= kFzSliceLds ? (int)slice : 0;
+    const size_t lds = area + sizeof(double) * (size_t)a.nslice;
+    const bool in = lds <= kFzLds;
+    const auto k = in ? (a.nft ? tci_floatingzone_kernel<true, true> : tci_floatingzone_kernel<true, false>)
+                      : (a.nft ? tci_floatingzone_kernel<false, true> : tci_floatingzone_kernel<false, false>);
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(256), in ? lds : 0, st, a);
     return hipGetLastError();
 }
 

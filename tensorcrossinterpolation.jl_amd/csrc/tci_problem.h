@@ -128,6 +128,19 @@ inline int check_functor(const tci_functor &f, int L, const int32_t *localdims, 
     return TCI_OK;
 }
 
+// most entries of a Gaussian sum's term tables (1 MiB)
+constexpr int kMaxTermTable = 1 << 17;
+
+// Sums over sites that f is made of (term_value): one for the weighted Lorentzian,
+// one per Gaussian of a Gaussian sum, while their tables stay small; else 0.
+inline int term_functions(const tci_functor &f, int L, int dmax)
+{
+    if (f.kind == TCI_F_LORENTZ_WEIGHTED) return 1;
+    if (f.kind == TCI_F_GAUSS_SUM && f.params[0] >= 1.0 && f.params[0] * (double)L * (double)dmax <= (double)kMaxTermTable)
+        return (int)f.params[0];
+    return 0;
+}
+
 // The key coefficients of the memo table (cachedfunction.jl:13-25):
 // coef_1 = 1, coef_i = d_{i-1}·coef_{i-1}, as 256-bit numbers (four 64-bit
 // limbs each, written to out when non-null).  False when the largest key,
@@ -214,8 +227,6 @@ inline int check_state(const tci_problem &p, std::string *msg)
     return TCI_OK;
 }
 
-// most entries of a Gaussian sum's term tables (1 MiB)
-constexpr int kMaxTermTable = 1 << 17;
 
 // Returns TCI_OK or an error with *msg set.
 inline int check_problem(const tci_problem &p, SolveCaps &c, std::string *msg)
@@ -279,13 +290,7 @@ inline int check_problem(const tci_problem &p, SolveCaps &c, std::string *msg)
     if (o.pivotsearch != 0 && o.pivotsearch != 1)
         return bad(TCI_ERR_ARG, "Unknown pivot search strategy. Choose from :rook, :full.");
     c.rook = o.pivotsearch;
-    // per-site terms of f (Engine::build_ftab): one table for the weighted
-    // Lorentzian, one per Gaussian of a Gaussian sum, while they stay small
-    c.nftab = 0;
-    if (p.f.kind == TCI_F_LORENTZ_WEIGHTED) c.nftab = 1;
-    if (p.f.kind == TCI_F_GAUSS_SUM && p.f.params[0] >= 1.0 &&
-        p.f.params[0] * (double)L * (double)dmax <= (double)kMaxTermTable)
-        c.nftab = (int32_t)p.f.params[0];
+    c.nftab = term_functions(p.f, L, dmax);
     return TCI_OK;
 }
 
