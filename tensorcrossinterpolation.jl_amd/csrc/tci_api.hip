@@ -1231,12 +1231,13 @@ static tci_status tt_download(TtDevice &T, int64_t *linkdims, double *cores)
 // per bond, the rrLU of the grouped site matrix, its left/right factors
 // (method 0 rrLU with permutations, 1 MatrixLUCI), the factored site
 // replaced by one of them and the other multiplied into the neighbour.
-// The whole sweep in one workgroup (launch_tt_sweep) for trains whose every
-// bond matrix holds at most kTtFusedElems entries: there the host-driven
-// sweep spends its time in per-bond round trips (about 80 us each), not in
-// the factorizations.  Same operations per entry, so the same bits.  Measured
-// (compress! of 20 sites, one workgroup / bond by bond, ms): 1024 entries 2.8 /
-// 3.3, 2304 4.5 / 5.3, 4096 7.3 / 6.1, 9216 15 / 7.5, 62 208 130 / 14.
+// The whole sweep in one workgroup (launch_tt_sweep) for trains whose bond
+// matrices hold at most kTtFusedElems entries in the mean and none more than
+// twice that: there the host-driven sweep spends its time in per-bond round trips
+// (about 80 us each), not in the factorizations.  Same operations per entry, so
+// the same bits.  Measured (compress!, one workgroup / bond by bond, ms): 20 sites
+// of 1024 entries 2.8 / 3.3, 2304 4.5 / 5.3, 4096 7.3 / 6.1, 9216 15 / 7.5, 62 208
+// 130 / 14; 40 uneven sites of at most 3136 9.7 / 11.1.
 constexpr int64_t kTtFusedElems = 3072;
 constexpr int64_t kTtStageCap = 48 * 1024 / 16;   // doubles per LDS staging vector
 constexpr int64_t kTtMatCap = 96 * 1024 / 8;       // doubles of LDS for a bond matrix
@@ -1320,14 +1321,15 @@ static tci_status tt_sweep(TtDevice &T, int32_t method, int32_t forward, int64_t
     int64_t R = 0;
     for (int b = 1; b < L; ++b) R = T.links[(size_t)b] > R ? T.links[(size_t)b] : R;
     {
-        int64_t big = 0;
+        int64_t big = 0, sum = 0;
         for (int b = 0; b + 1 < L; ++b) {
             const int64_t mm = forward ? T.links[(size_t)b] * T.d[(size_t)b] : T.links[(size_t)b + 1];
             const int64_t nn = forward ? T.links[(size_t)b + 1] : T.d[(size_t)b + 1] * T.links[(size_t)b + 2];
             big = mm * nn > big ? mm * nn : big;
+            sum += mm * nn;
         }
         const char *ev = getenv("TCI_TT_FUSED");
-        const bool fused = ev ? atoi(ev) != 0 : big <= kTtFusedElems;
+        const bool fused = ev ? atoi(ev) != 0 : big <= 2 * kTtFusedElems && sum <= kTtFusedElems * (L - 1);
         if (fused && L > 1 && R > 0) return tt_sweep_fused(T, method, forward, maxrank, reltol, abstol, R, pivots, pivoterrors);
     }
     if (pivoterrors)

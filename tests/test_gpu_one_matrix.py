@@ -98,8 +98,8 @@ def test_product(tci, ctx, M, N, K):
     assert np.array_equal(np.signbit(out[num]), np.signbit(ref[num]))
 
 
-# the largest bond matrix just under, at and above the fused sweep's limit
-@pytest.mark.parametrize("chi,d", [(32, 2), (32, 3), (33, 3), (55, 1)])
+# bond matrices just under, at and above the fused sweep's limits, in the mean and the largest
+@pytest.mark.parametrize("chi,d", [(32, 2), (32, 3), (33, 3), (55, 1), (47, 2), (48, 2), (56, 2)])
 @pytest.mark.parametrize("method", ["LU", "CI"])
 def test_sweep_limit(tci, ctx, chi, d, method):
     cores = random_tt([1, chi, chi, chi, 1], [d] * 4, chi + d)[2]
