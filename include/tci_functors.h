@@ -87,7 +87,7 @@ static inline TCI_HD double tci_pow2i(int k)
 static inline TCI_HD double tci_round_half_away(double x)
 {
     /* nearest integer, ties away from zero; |x| < 2^52 */
-    return x >= 0.0 ? (double)(int64_t)(x + 0.5) : -(double)(int64_t)(0.5 - x);
+    return x >= 0.0 ? __builtin_trunc(x + 0.5) : -__builtin_trunc(0.5 - x);
 }
 
 /* exp(x): x = k·ln2 + r with ln2 split as hi (42 significant bits, so k·hi
@@ -98,12 +98,13 @@ static inline TCI_HD double tci_exp(double x)
     const double LN2_HI = 0.6931471805598903;        /* bits 0x3fe62e42fefa3800 */
     const double LN2_LO = 5.497923018708371e-14;     /* ln2 - LN2_HI */
     const double INV_LN2 = 1.4426950408889634;
-    if (x != x) return x;
-    if (x > 709.782712893384) return 1.0 / 0.0;
-    if (x < -745.1332191019412) return 0.0;
-    double kd = tci_round_half_away(x * INV_LN2);
+    /* no branches, so that several values run side by side: the result is selected
+     * at the end, and 2^k taken in two factors, one of them 1 unless k is beyond the
+     * normal exponents */
+    const double y = x >= -745.1332191019412 && x <= 709.782712893384 ? x : 0.0;
+    double kd = tci_round_half_away(y * INV_LN2);
     int k = (int)kd;
-    double r = (x - kd * LN2_HI) - kd * LN2_LO;
+    double r = (y - kd * LN2_HI) - kd * LN2_LO;
     /* Horner on Σ_{n=0}^{15} r^n / n! */
     double p = 7.647163731819816e-13;                /* 1/15! */
     p = p * r + 1.1470745597729725e-11;              /* 1/14! */
@@ -121,11 +122,11 @@ static inline TCI_HD double tci_exp(double x)
     p = p * r + 0.5;                                 /* 1/2!  */
     p = p * r + 1.0;
     p = p * r + 1.0;
-    if (k >= -1022) {
-        if (k <= 1023) return p * tci_pow2i(k);
-        return (p * tci_pow2i(1023)) * tci_pow2i(k - 1023);
-    }
-    return (p * tci_pow2i(k + 1000)) * tci_pow2i(-1000);
+    const int k1 = k > 1023 ? 1023 : k < -1022 ? k + 1000 : k;
+    p = (p * tci_pow2i(k1)) * tci_pow2i(k > 1023 ? k - 1023 : k < -1022 ? -1000 : 0);
+    p = x > 709.782712893384 ? 1.0 / 0.0 : p;
+    p = x < -745.1332191019412 ? 0.0 : p;
+    return x != x ? x : p;
 }
 
 /* sin(r), cos(r) for |r| <= π/4 by Taylor series (to r^17 / r^18). */
