@@ -43,9 +43,41 @@
 // (512 threads, 4×18 doubles a lane).
 #pragma once
 
+#include <type_traits>
+#include <utility>
+
 #include "tci_common.h"
 
 namespace tci {
+
+// What a team offers beyond the basic interface: a team with best_slot has two sets
+// of slots (tA, tB and tX take wave + NW·parity) and reduces a set by itself.  A team
+// without it has NW slots; a step then costs a second barrier, before the slots are
+// written again, and the slots are compared one by one.
+template <class Team, class = void>
+struct TileSlots {
+    static constexpr int SETS = 1;
+    ENG_INLINE static int best(Team &tm, int at, uint32_t &K)
+    {
+        double g = -1.0;
+        for (int q = 0; q < Team::NW; ++q) g = tm.tA(at + q) > g ? tm.tA(at + q) : g;
+        K = 0xffffffffu;
+        int w = 0;
+        for (int q = 0; q < Team::NW; ++q) {
+            const double v = tm.tA(at + q);
+            if (v >= 0.0 && v * v == g * g && tm.tB(at + q) < K) {
+                K = tm.tB(at + q);
+                w = q;
+            }
+        }
+        return w;
+    }
+};
+template <class Team>
+struct TileSlots<Team, std::void_t<decltype(std::declval<Team &>().best_slot(0, std::declval<uint32_t &>()))>> {
+    static constexpr int SETS = 2;
+    ENG_INLINE static int best(Team &tm, int at, uint32_t &K) { return tm.best_slot(at, K); }
+};
 
 template <class Team, int RA, int CB, bool EX = false>
 struct TileLU {
@@ -349,7 +381,8 @@ struct TileLU {
 #else
         constexpr bool vote = WS == 1;
 #endif
-        par ^= 1;
+        if constexpr (TileSlots<Team>::SETS == 2) par ^= 1;
+        else tm.sync();   // (every wave has read the last search's slots)
         const int me = tm.wave() + NW * par;
         double lmax = ex;
 #pragma unroll
@@ -447,7 +480,7 @@ struct TileLU {
         }
         tm.sync();
         uint32_t K;
-        const int w = tm.best_slot(NW * par, K);
+        const int w = TileSlots<Team>::best(tm, NW * par, K);
         wstar = w + NW * par;
         return K;
     }
