@@ -225,7 +225,7 @@ __device__ __forceinline__ bool chip_job(const ChipArgs &K, ChipLds<NW> &sh, dou
     const auto excol = [&](int e) { return g + S * (CB + e); };
     // a thread's column maximum cm joins the running maximum; emask keeps the
     // columns within 2^-50 of it (entries of equal squares are closer than that
-    // unless the square is subnormal, where every column is scanned)
+    // unless the square is subnormal or infinite, where every column is scanned)
     const auto emax = [&](int e, double cm) {
         if (cm > lmaxe) {
             emask = lmaxe >= cm * (1.0 - 0x1p-50) ? emask | (1ULL << e) : 1ULL << e;
@@ -298,7 +298,7 @@ __device__ __forceinline__ bool chip_job(const ChipArgs &K, ChipLds<NW> &sh, dou
             }
             if (EX) {
                 const bool minee = lmaxe * lmaxe == G && lmaxe >= 0.0;
-                const bool all = !(G >= 0x1p-1022);   // a subnormal square
+                const bool all = !(G >= 0x1p-1022 && G < __builtin_inf());   // (emask does not tell)
                 for (int e = 0; e < nex; ++e) {
                     if (!tm.wave_any(minee && (all || ((emask >> e) & 1)))) continue;
                     const int c = sh.ecp[e];
