@@ -85,6 +85,7 @@ struct tci_ctx {
     int rrlu_algo = TCI_RRLU_AUTO;   // factorization kernel of the standalone rrLU
     std::vector<tci_rrlu_tune> tune; // measured AUTO choices (tci_ctx_autotune_rrlu), by side
     int ncu = 0;                     // compute units
+    uint64_t chip_wait = 60000000000ULL;   // longest wait of an on-chip rrLU's member (TCI_RRLU_WAIT_MS; 600 s)
     std::vector<uint8_t> chip_host, tile_host;   // host copies of the last rrLU's tables
 };
 
@@ -377,6 +378,10 @@ tci_status tci_ctx_create(tci_ctx **out, int32_t device, uint64_t hbm_budget_byt
     c->team = ev ? atoi(ev) : 256;
     c->team_env = ev != nullptr;
     if (c->team != 64 && c->team != 256 && c->team != 512 && c->team != 1024) c->team = 256;
+    // (a member may have to wait for workgroups that another stream's kernels keep
+    // from starting; 0: any wait is given up)
+    ev = getenv("TCI_RRLU_WAIT_MS");
+    if (ev && atoll(ev) >= 0) c->chip_wait = (uint64_t)atoll(ev) * 100000;
     ev = getenv("TCI_WG_PER_CU");
     c->wg_env = ev && atoi(ev) > 0 ? atoi(ev) : 0;
     HIPCHK(hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, device));
@@ -623,6 +628,7 @@ static tci_status lu_run_chip(tci_ctx *ctx, tci_lu_job *jobs, const LuPlan &P, s
     K.abort_word = (uint32_t *)(z + 128);
     K.mail = (uint64_t *)(z + 256);
     K.cols = (double *)(z + b_mail);
+    K.wait_ticks = ctx->chip_wait;
     K.colcap = colcap;
     K.spill = (double *)(z + b_mail + b_cols);
     K.spillcap = spill;

@@ -88,7 +88,8 @@ struct ChipArgs {
     const int32_t *map;      // ticket → item
     int32_t ntickets;
     uint32_t *ticket;        // next ticket (zero on entry)
-    uint32_t *abort_word;    // zero on entry
+    uint32_t *abort_word;    // zero on entry; not zero: a member has given up a wait
+    uint64_t wait_ticks;     // the longest wait (100 MHz wall clock)
     uint64_t *mail;          // 8 words per ticket (zero on entry)
     double *cols;            // 2 × colcap per workgroup (rrlu_chip_blocks of them)
     int64_t colcap;          // rows of the tallest job

@@ -42,7 +42,9 @@
 // later than any ticket after them, so the earliest unfinished job always
 // finishes as long as the largest team fits the device at once (the launch is
 // cooperative, so the whole grid does).  Every wait is bounded all the same: a
-// member that waits longer than kChipWaitTicks gives up and tells the others.
+// member that waits longer than ChipArgs::wait_ticks gives up and tells the others.
+// The workgroups go on drawing tickets: every job whose team has given up, and every
+// team's job drawn after that, reports TCI_ERR_DEVICE, so no job is left as it was.
 //
 // tci_rrlu_chip_kernel runs two workgroups of four waves per CU, one of them
 // working while the other waits for its team.  Matrices that need more
@@ -66,15 +68,13 @@
 
 namespace tci {
 
-// 600 s of the 100 MHz wall clock: a member may have to wait for workgroups that
-// another stream's kernels keep from starting
-constexpr uint64_t kChipWaitTicks = 60000000000ULL;
 constexpr int kChipMaxCB = 42;
 constexpr int kChipMaxExtra = 64;                    // columns of a member outside its registers
 constexpr int kChipColLds = 1024;                    // rows of a lone member's column kept in LDS
 constexpr int kChipL2Share = 14000;                  // doubles of L2 a member of the big kernel may count on
 constexpr uint32_t kChipNone = 0xffffffffu;
 constexpr int kChipOut = 0xffff;                     // position of a row or column that does not exist
+constexpr int kChipFail = 3;                         // word of member 0's mailbox: a member has given up
 
 // Pointers into device memory carry their address space: through generic ones
 // every access would also count as an LDS operation, and each barrier would wait
@@ -122,9 +122,11 @@ __device__ __forceinline__ void mail_put(GU64 *s, double a, uint32_t key, uint32
 }
 
 // waits for a member's mailbox of this round; false when the wait was given up
-__device__ __forceinline__ bool mail_get(const GU64 *s, uint32_t round, GU32 *abort_word, double &a,
+__device__ __forceinline__ bool mail_get(const GU64 *s, uint32_t round, const ChipArgs &K, double &a,
                                          uint32_t &key, uint32_t &blk)
 {
+    GU32 *abort_word = (GU32 *)K.abort_word;
+    const uint32_t every = K.wait_ticks ? 0xfffu : 0u;   // polls between looks at the clock
     uint64_t t0 = 0;
     for (uint32_t spin = 0;; ++spin) {
         const uint64_t w0 = agent_get(s), w1 = agent_get(s + 1), w2 = agent_get(s + 2);
@@ -134,14 +136,23 @@ __device__ __forceinline__ bool mail_get(const GU64 *s, uint32_t round, GU32 *ab
             blk = (uint32_t)(w2 >> 26) & 0x3ffu;
             return true;
         }
-        if ((spin & 0xfffu) == 0xfffu) {
+        if ((spin & every) == every) {
             const uint64_t now = (uint64_t)wall_clock64();
             if (t0 == 0) t0 = now;
-            if (now - t0 > kChipWaitTicks)
+            if (now - t0 >= K.wait_ticks)
                 __hip_atomic_store(abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (__hip_atomic_load(abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return false;
         }
     }
+}
+
+// A job's status and rank, written past this XCD's L2 and acknowledged: members on
+// several XCDs may write them (chip_failed)
+__device__ __forceinline__ void job_put(tci_lu_job &J, int32_t status, int64_t npivot)
+{
+    __hip_atomic_store((GI32 *)&J.status, status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    agent_put((GU64 *)&J.npivot, (uint64_t)npivot);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 // One member's part of one job.  EX: columns beyond the registers are kept in
@@ -167,7 +178,6 @@ __device__ __forceinline__ bool chip_job(const ChipArgs &K, ChipLds<NW> &sh, dou
     const uint32_t me = blockIdx.x;
     const int m = (int)J.m, n = (int)J.n;
     GDbl *__restrict__ A = (GDbl *)J.A;
-    GU32 *abort_word = (GU32 *)K.abort_word;
     const bool lo = J.leftorth != 0;
     const double reltol = J.reltol, abstol = J.abstol;
     int mr = m < n ? m : n;
@@ -397,7 +407,7 @@ __device__ __forceinline__ bool chip_job(const ChipArgs &K, ChipLds<NW> &sh, dou
             for (int q = tid; q < S; q += NT) {
                 double qa;
                 uint32_t qk, qb;
-                if (!mail_get(mail + (int64_t)8 * q + 4 * par, seen + 1, abort_word, qa, qk, qb)) {
+                if (!mail_get(mail + (int64_t)8 * q + 4 * par, seen + 1, K, qa, qk, qb)) {
                     sh.abort = 1;
                     break;
                 }
@@ -642,7 +652,7 @@ __device__ __forceinline__ bool chip_job(const ChipArgs &K, ChipLds<NW> &sh, dou
         for (int q = tid; q < S; q += NT) {
             double qa;
             uint32_t qk, qb;
-            if (!mail_get(mail + (int64_t)8 * q + 4 * par, seen + 1, abort_word, qa, qk, qb)) {
+            if (!mail_get(mail + (int64_t)8 * q + 4 * par, seen + 1, K, qa, qk, qb)) {
                 sh.abort = 1;
                 break;
             }
@@ -682,22 +692,25 @@ __device__ __forceinline__ bool chip_job(const ChipArgs &K, ChipLds<NW> &sh, dou
         }
         if (tid == 0) {
             // lu.L is checked first (matrixlu.jl:164-169)
-            J.status = nanL ? TCI_ERR_NAN_L : nanU ? TCI_ERR_NAN_U : TCI_OK;
-            J.npivot = nanL || nanU ? 0 : p;
+            job_put(J, nanL ? TCI_ERR_NAN_L : nanU ? TCI_ERR_NAN_U : TCI_OK, nanL || nanU ? 0 : p);
             J.error = p >= (m < n ? m : n) ? 0.0 : err;
+            // a member that gave up in the last exchange: it marks the team's fail word
+            // and then the job, so either this sees the mark or its status comes last
+            if (S > 1 && agent_get(mail + kChipFail)) job_put(J, TCI_ERR_DEVICE, 0);
         }
     }
     return true;
 }
 
-// the next ticket's job and this workgroup's place in its team; false: none left
+// the next ticket's job and this workgroup's place in its team; false: none left.
+// sh.abort: the launch has given up (a lone member's job is still done)
 template <int NW>
 __device__ __forceinline__ bool chip_draw(const ChipArgs &K, ChipLds<NW> &sh, ChipItem &it, int &g)
 {
     __syncthreads();   // the last job's shared data is done with
     if (threadIdx.x == 0) {
         sh.ticket = (int32_t)__hip_atomic_fetch_add(K.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        sh.abort = 0;
+        sh.abort = (int32_t)__hip_atomic_load(K.abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
     const int t = __builtin_amdgcn_readfirstlane(sh.ticket);
@@ -707,11 +720,15 @@ __device__ __forceinline__ bool chip_draw(const ChipArgs &K, ChipLds<NW> &sh, Ch
     return true;
 }
 
-__device__ __forceinline__ void chip_failed(tci_lu_job &J)
+// a member that gave up on the ticket drawn last: its team's fail word, then its job
+// (looked up again, so that the register shapes need not hold it)
+__device__ __forceinline__ void chip_failed(const ChipArgs &K, int ticket)
 {
     if (threadIdx.x == 0) {
-        J.status = TCI_ERR_DEVICE;
-        J.npivot = 0;
+        const ChipItem it = K.items[K.map[ticket]];
+        agent_put((GU64 *)K.mail + (int64_t)8 * it.first + kChipFail, 1);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        job_put(K.jobs[it.job], TCI_ERR_DEVICE, 0);
     }
 }
 
@@ -727,7 +744,8 @@ __global__ __launch_bounds__(256, 2) void tci_rrlu_chip_kernel(ChipArgs K)
         tci_lu_job &J = K.jobs[it.job];
         GU64 *mail = (GU64 *)K.mail + (int64_t)8 * it.first;
         bool ok = true;
-        switch (it.shape) {
+        if (it.S > 1 && sh.abort) ok = false;
+        else switch (it.shape) {
         case 0: ok = chip_job<4, 2, 42, false>(K, sh, nullptr, 0, J, it.S, g, it.wr, mail); break;
         case 1: ok = chip_job<4, 3, 28, false>(K, sh, nullptr, 0, J, it.S, g, it.wr, mail); break;
         case 2: ok = chip_job<4, 4, 22, false>(K, sh, nullptr, 0, J, it.S, g, it.wr, mail); break;
@@ -736,10 +754,7 @@ __global__ __launch_bounds__(256, 2) void tci_rrlu_chip_kernel(ChipArgs K)
         case 5: ok = chip_job<4, 8, 10, false>(K, sh, nullptr, 0, J, it.S, g, it.wr, mail); break;
         default: ok = chip_job<4, 12, 6, false>(K, sh, nullptr, 0, J, it.S, g, it.wr, mail); break;
         }
-        if (!ok) {
-            chip_failed(J);
-            return;
-        }
+        if (!ok) chip_failed(K, sh.ticket);
     }
 }
 
@@ -753,16 +768,14 @@ __global__ __launch_bounds__(512, 2) void tci_rrlu_chip_big_kernel(ChipArgs K, i
         tci_lu_job &J = K.jobs[it.job];
         GU64 *mail = (GU64 *)K.mail + (int64_t)8 * it.first;
         bool ok = true;
-        switch (it.shape) {
+        if (it.S > 1 && sh.abort) ok = false;
+        else switch (it.shape) {
         case 0: ok = chip_job<8, 6, 12, true>(K, sh, exl, exl_cap, J, it.S, g, 8, mail); break;
         case 1: ok = chip_job<8, 9, 9, true>(K, sh, exl, exl_cap, J, it.S, g, 8, mail); break;
         case 2: ok = chip_job<8, 12, 6, true>(K, sh, exl, exl_cap, J, it.S, g, 8, mail); break;
         default: ok = chip_job<8, 16, 4, true>(K, sh, exl, exl_cap, J, it.S, g, 8, mail); break;
         }
-        if (!ok) {
-            chip_failed(J);
-            return;
-        }
+        if (!ok) chip_failed(K, sh.ticket);
     }
 }
 
