@@ -87,6 +87,7 @@ struct tci_ctx {
     int ncu = 0;                     // compute units
     uint64_t chip_wait = 60000000000ULL;   // longest wait of an on-chip rrLU's member (TCI_RRLU_WAIT_MS; 600 s)
     std::vector<uint8_t> chip_host, tile_host;   // host copies of the last rrLU's tables
+    bool lu_queued = false;          // their uploads, or lu_order's, may still be queued on the stream
 };
 
 // a device-to-host copy of a finished result on the context's download
@@ -415,6 +416,7 @@ tci_status tci_ctx_synchronize(tci_ctx *ctx)
 {
     if (!ctx) return set_err(TCI_ERR_ARG, "ctx is NULL");
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    ctx->lu_queued = false;
     for (hipStream_t s : ctx->extra) HIPCHK(hipStreamSynchronize(s));
     return TCI_OK;
 }
@@ -487,6 +489,14 @@ struct LuPlan {
 
 static tci_status lu_partition(tci_ctx *ctx, int64_t tile_budget, LuPlan &P, bool allow_chip = true);
 
+// waits for the context's first stream: the rrLU's host tables are free again
+static hipError_t lu_wait(tci_ctx *ctx)
+{
+    const hipError_t e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) ctx->lu_queued = false;
+    return e;
+}
+
 // While a serving grid is resident on the device a cooperative launch waits for
 // it to leave, so then the on-chip kernels take only jobs of at least this many
 // elements, and those only when a batch has at most kGridMaxJobs of them
@@ -500,7 +510,7 @@ static tci_status lu_read(tci_ctx *ctx, tci_lu_job *jobs, int64_t count, LuPlan 
     P.h.resize((size_t)count);
     HIPCHK(hipMemcpyAsync(P.h.data(), jobs, sizeof(tci_lu_job) * (size_t)count, hipMemcpyDeviceToHost,
                           ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    HIPCHK(lu_wait(ctx));
     for (const tci_lu_job &j : P.h) {
         if (j.m < 0 || j.n < 0 || j.m > INT32_MAX / 2 || j.n > INT32_MAX / 2 || j.m * j.n > ((int64_t)1 << 31))
             return set_err(TCI_ERR_ARG, "job shape out of range");
@@ -605,9 +615,8 @@ static tci_status lu_run_chip(tci_ctx *ctx, tci_lu_job *jobs, const LuPlan &P, s
     const size_t b_mail = lay_align((size_t)64 * (size_t)nt) + 256;
     const size_t b_cols = lay_align(sizeof(double) * 2 * (size_t)colcap * (size_t)blocks);
     const size_t b_spill = sizeof(double) * (size_t)spill * (size_t)blocks;
-    // (the host copy lives in the context: the next call on this stream
-    // synchronizes before it reuses it)
     std::vector<uint8_t> &h = ctx->chip_host;
+    ctx->lu_queued = true;
     h.resize(b_items + b_map);
     memcpy(h.data(), items.data(), sizeof(ChipItem) * items.size());
     int32_t *map = (int32_t *)(h.data() + b_items);
@@ -663,17 +672,18 @@ static void stream_order(const LuPlan &P, std::vector<int32_t> &order)
 constexpr int64_t kLuLdsStageCap = 48 * 1024 / 16;   // doubles per staging vector in LDS
 
 // The launches of a batch whose jobs are known on the host (P.h), jobs their
-// device table.  The tables of each kernel go up from memory of the context: a
-// caller has synchronized the stream since the last call that used it.
+// device table.  The tables of each kernel go up from memory of the context, so an
+// earlier call's uploads are waited for if nothing has done so since.
 static tci_status lu_launch(tci_ctx *ctx, tci_lu_job *jobs, LuPlan &P)
 {
     const int64_t count = (int64_t)P.h.size();
     tci_status ps = lu_partition(ctx, -1, P);
     if (ps != TCI_OK) return ps;
     std::vector<int32_t> &tile = P.tile, &stream = P.stream;
+    if (ctx->lu_queued) HIPCHK(lu_wait(ctx));
     ps = lu_run_chip(ctx, jobs, P, P.chip, 0);
     if (ps != TCI_OK) return ps;
-    if (!P.chip.empty() && !P.big.empty()) HIPCHK(hipStreamSynchronize(ctx->stream));   // (chip_host is used again)
+    if (!P.chip.empty() && !P.big.empty()) HIPCHK(lu_wait(ctx));   // (chip_host is used again)
     ps = lu_run_chip(ctx, jobs, P, P.big, 1);
     if (ps != TCI_OK) return ps;
     if (!tile.empty()) {
@@ -681,6 +691,7 @@ static tci_status lu_launch(tci_ctx *ctx, tci_lu_job *jobs, LuPlan &P)
         const size_t b_idx = lay_align(sizeof(int32_t) * tile.size());
         const size_t b_off = lay_align(sizeof(int64_t) * P.soff.size());
         std::vector<uint8_t> &h = ctx->tile_host;
+        ctx->lu_queued = true;
         h.resize(b_idx + b_off);
         memcpy(h.data(), tile.data(), sizeof(int32_t) * tile.size());
         memcpy(h.data() + b_idx, P.soff.data(), sizeof(int64_t) * P.soff.size());
@@ -697,6 +708,7 @@ static tci_status lu_launch(tci_ctx *ctx, tci_lu_job *jobs, LuPlan &P)
     double *gstage = nullptr;
     if (mx > kLuLdsStageCap) HIPCHK(hipMallocAsync((void **)&gstage, sizeof(double) * 2 * mx * count, ctx->stream));
     std::vector<int32_t> &order = ctx->lu_order;
+    ctx->lu_queued = true;
     stream_order(P, order);
     const int64_t ns = (int64_t)order.size();
     int32_t *dorder = nullptr;
@@ -795,7 +807,7 @@ static tci_status lu_one(tci_ctx *ctx, const double *A, int64_t lda, int64_t m, 
         // (U starts where L of the rank found ends: the kernel packs them)
         e = launch_lu_unpack((const tci_lu_job *)djob, (m + n + 1) * cap, dL, nullptr, nullptr, nullptr, st);
     if (e == hipSuccess && s == TCI_OK) e = hipMemcpyAsync(h, djob, down, hipMemcpyDeviceToHost, st);
-    const hipError_t es = hipStreamSynchronize(st);
+    const hipError_t es = lu_wait(ctx);
     if (e == hipSuccess) e = es;
     if (e == hipSuccess && s == TCI_OK) {
         memcpy(&j, h, sizeof j);
@@ -1372,7 +1384,7 @@ static tci_status tt_sweep(TtDevice &T, int32_t method, int32_t forward, int64_t
         HIPCHK(launch_lu_unpack(T.job, (m + n + 1) * std::min(m, n), T.wl, T.wu, T.diag,
                                 method == 1 && !forward ? T.wt : nullptr, st));
         HIPCHK(hipMemcpyAsync(T.hres, T.job, T.res_bytes, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
+        HIPCHK(lu_wait(ctx));
         memcpy(&j, T.hres, sizeof j);
         if (j.status == TCI_ERR_NAN_L) return set_err(TCI_ERR_NAN_L, "lu.L contains NaNs");
         if (j.status == TCI_ERR_NAN_U) return set_err(TCI_ERR_NAN_U, "lu.U contains NaNs");
