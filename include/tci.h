@@ -176,9 +176,9 @@ tci_status tci_ctx_set_rrlu_algo(tci_ctx *ctx, int32_t algo);
  * the context, and AUTO then follows them: a job of largest side s uses the
  * first entry whose side is at least s (the last one beyond it).  The
  * register tile is used when that entry's tile is set.  The cooperative
- * kernel is used when the batch holds no more such jobs than every one of
- * their entries' grid_max_jobs.  Choices change
- * speed only: every kernel gives the same bits.  Writes up to cap entries
+ * kernel is used when the batch holds no more such jobs of that entry than
+ * its grid_max_jobs; 64, the most that is timed, or more sets no limit.
+ * Choices change speed only: every kernel gives the same bits.  Writes up to cap entries
  * to table (may be NULL) and their number to *count.  Takes a few seconds
  * and up to about 9 GB of the HBM budget while it runs.
  * tci_ctx_set_rrlu_tuning installs a table (one measured earlier and saved);
@@ -189,7 +189,8 @@ typedef struct tci_rrlu_tune {
     int32_t grid_team;       /* threads per workgroup of the cooperative kernel that
                                 takes this side (256 or 512 when measured; 256, 512
                                 and 1024 are accepted, the kernel goes by the shape) */
-    int32_t grid_max_jobs;   /* most such jobs the cooperative kernel takes (0: none) */
+    int32_t grid_max_jobs;   /* most such jobs the cooperative kernel takes in one batch
+                                (0: none, 64 and more: any number) */
     float ms_stream;         /* one matrix, streaming kernel                   */
     float ms_grid;           /* one matrix, cooperative kernel                 */
     float ms_tile_batch;     /* 512 matrices, register tile (side <= 128)      */
