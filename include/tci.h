@@ -413,7 +413,9 @@ tci_status tci_batch_sitetensor(tci_batch *b, int32_t i, int32_t site, int64_t *
  * valid until tci_batch_free.  tdims: 3·L, the dims3 of every site; tensors:
  * the site tensors back to back; counts: 4·L, counts[which·L + site-1] as
  * tci_batch_indexset gives them; sets: the entries back to back, in the order
- * which, site, entry. */
+ * which, site, entry.  The first piece asked of a solve may bring up to three
+ * others' results into host memory for each one read before; device memory is
+ * taken only as far as the HBM budget has it left. */
 tci_status tci_batch_solution(tci_batch *b, int32_t i, const int64_t **tdims, const double **tensors,
                               const int32_t **counts, const uint8_t **sets);
 tci_status tci_batch_pivoterrors(tci_batch *b, int32_t i, double *out, int64_t cap);

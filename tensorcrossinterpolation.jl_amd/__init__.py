@@ -956,16 +956,18 @@ def crossinterpolate2_batch(problems, ctx=None, return_batch=False, error_sample
         retry = []
         try:
             _check(lib.tci_batch_wait(b))
+            r = _abi.tci_result()
             for k, i in enumerate(pending):
-                t = TensorCI2(b, k, problems[i][1])
+                _check(lib.tci_batch_result(b, k, C.byref(r)))
                 user_cap = int(problems[i][3].get("chi_cap", 0) or 0)
-                if t.status == 10 and user_cap == 0:
+                if r.status == 10 and user_cap == 0:
                     used, limit = capacity_plan(holders[k])
                     if used < limit:
                         chi[i] = int(min(2 * used, limit, 8192))
                         if chi[i] > used:
                             retry.append(i)
                             continue
+                t = TensorCI2(b, k, problems[i][1])
                 if error_sample and t.status == 0:
                     npts, seed = error_sample
                     x = sample_points(problems[i][1], int(npts), seed)

@@ -56,6 +56,7 @@ static tci_status set_err(tci_status code, const char *fmt, ...)
 struct PoolBuf {
     void *ptr;
     size_t bytes;
+    bool pinned = true;   // host buffers: ordinary memory where pinning failed
 };
 
 struct tci_ctx {
@@ -196,7 +197,8 @@ static void pool_put(tci_ctx *c, void *p, size_t bytes)
 }
 
 // Pinned host buffers of packed results, kept between batches (pinning costs
-// more than the download): up to kHostPoolBytes in at most kHostPoolBufs buffers
+// more than the download): up to kHostPoolBytes in at most kHostPoolBufs buffers.
+// Where no memory can be pinned, ordinary memory, which is only slower
 constexpr size_t kHostPoolBytes = (size_t)512 << 20;
 constexpr size_t kHostPoolBufs = 8;
 
@@ -209,14 +211,24 @@ static hipError_t hpool_get(tci_ctx *c, size_t bytes, PoolBuf *out)
             return hipSuccess;
         }
     out->bytes = bytes;
-    return hipHostMalloc(&out->ptr, bytes, hipHostMallocDefault);
+    out->pinned = hipHostMalloc(&out->ptr, bytes, hipHostMallocDefault) == hipSuccess;
+    if (out->pinned) return hipSuccess;
+    (void)hipGetLastError();
+    out->ptr = malloc(bytes);
+    return out->ptr ? hipSuccess : hipErrorOutOfMemory;
+}
+
+static void host_free(const PoolBuf &b)
+{
+    if (b.pinned) (void)hipHostFree(b.ptr);
+    else free(b.ptr);
 }
 
 static void hpool_put(tci_ctx *c, const PoolBuf &b)
 {
     size_t tot = b.bytes;
     for (const PoolBuf &q : c->hpool) tot += q.bytes;
-    if (tot > kHostPoolBytes || c->hpool.size() >= kHostPoolBufs) (void)hipHostFree(b.ptr);
+    if (!b.pinned || tot > kHostPoolBytes || c->hpool.size() >= kHostPoolBufs) host_free(b);
     else c->hpool.push_back(b);
 }
 
@@ -268,7 +280,7 @@ struct tci_batch {
     };
     std::vector<Packed> packed;
     std::vector<PoolBuf> packs;            // their pinned buffers
-    std::vector<std::vector<uint8_t>> hostpacks;   // of served requests: ordinary memory
+    std::vector<std::vector<uint8_t>> hostpacks;   // read piece by piece: ordinary memory
     int npacked = 0;
 };
 
@@ -405,7 +417,7 @@ tci_status tci_ctx_destroy(tci_ctx *ctx)
         (void)hipStreamDestroy(s);
     }
     for (PoolBuf &b : ctx->pool) (void)hipFree(b.ptr);
-    for (PoolBuf &b : ctx->hpool) (void)hipHostFree(b.ptr);
+    for (PoolBuf &b : ctx->hpool) host_free(b);
     (void)hipStreamDestroy(ctx->dl);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -1619,7 +1631,7 @@ static void batch_release(tci_batch *b)
     if (b->ev1) (void)hipEventDestroy(b->ev1);
     for (const PoolBuf &q : b->packs) {
         if (b->ctx) hpool_put(b->ctx, q);
-        else (void)hipHostFree(q.ptr);
+        else host_free(q);
     }
     delete b;
 }
@@ -1957,70 +1969,84 @@ static size_t pack_shape(const SolveDesc &R, tci_batch::Packed &P, size_t *tenso
     return (size_t)o + (((size_t)s + 15) & ~(size_t)15);
 }
 
-constexpr size_t kPackGroupBytes = (size_t)1 << 30;
-
-// Solve i's site tensors and index sets in host memory.  The first solve asked
-// for is packed alone; when another one follows, all the others come with it (a
-// download per tensor and set costs 25 us each, and a batch of 384 solves has
-// 15 000 of them: 640 ms against 3 for the solves themselves), up to 1 GiB at a
-// time.  A served request is read directly: its pack kernel could have to wait
-// for the resident grid.
-static tci_status ensure_packed(tci_batch *b, int32_t i)
+// Single pieces of a solve's results, by downloads of their own: one site tensor,
+// and one index set's entries
+static tci_status direct_tensor(tci_ctx *ctx, const SolveDesc &R, int b0, int64_t n, void *out)
 {
-    SolveDesc R;
-    if (!report_view(b, i, R)) return set_err(TCI_ERR_ARG, "bad batch/index");
-    if (b->packed.empty()) b->packed.resize((size_t)b->count);
-    if (!b->packed[(size_t)i].counts.empty()) return TCI_OK;
-    tci_ctx *ctx = b->ctx;
-    HIPCHK(hipSetDevice(ctx->device));
+    HIPCHK(ctx_download(ctx, out, R.T + R.tstride * b0, sizeof(double) * (size_t)n));
+    return TCI_OK;
+}
+static tci_status direct_set(tci_ctx *ctx, const SolveDesc &R, int which, int b0, int cnt, int len, uint8_t *out)
+{
+    std::vector<uint8_t> raw((size_t)cnt * R.L);
+    HIPCHK(ctx_download(ctx, raw.data(), R.sets + ((int64_t)(set_kind(R, which) * R.L + b0) * R.setcap) * R.L,
+                        raw.size()));
+    for (int e = 0; e < cnt; ++e) memcpy(out + (size_t)e * len, raw.data() + (size_t)e * R.L, (size_t)len);
+    return TCI_OK;
+}
+
+// solve i's results read piece by piece
+static tci_status direct_solution(tci_batch *b, int32_t i, const SolveDesc &R)
+{
+    tci_batch::Packed P;
     size_t tb = 0;
-    if (b->served) {
-        tci_batch::Packed P;
-        const size_t bytes = pack_shape(R, P, &tb);
-        std::vector<uint8_t> h(bytes ? bytes : 1);
-        std::vector<uint8_t> raw;
-        for (int s = 0; s < R.L; ++s) {
-            const int64_t n = P.tdims[(size_t)3 * s] * P.tdims[(size_t)3 * s + 1] * P.tdims[(size_t)3 * s + 2];
-            if (n > 0) HIPCHK(ctx_download(ctx, h.data() + P.off[(size_t)5 * s], R.T + R.tstride * s, sizeof(double) * n));
-            for (int w = 0; w < 4; ++w) {
-                const int cnt = P.counts[(size_t)w * R.L + s], len = set_len(R, w, s);
-                if (cnt == 0 || len == 0) continue;
-                raw.resize((size_t)cnt * R.L);
-                const uint8_t *src = R.sets + ((int64_t)(set_kind(R, w) * R.L + s) * R.setcap) * R.L;
-                HIPCHK(ctx_download(ctx, raw.data(), src, raw.size()));
-                uint8_t *dst = h.data() + tb + P.off[(size_t)5 * s + 1 + w];
-                for (int e = 0; e < cnt; ++e) memcpy(dst + (size_t)e * len, raw.data() + (size_t)e * R.L, (size_t)len);
-            }
+    const size_t bytes = pack_shape(R, P, &tb);
+    std::vector<uint8_t> h(bytes ? bytes : 1);
+    for (int s = 0; s < R.L; ++s) {
+        const int64_t n = P.tdims[(size_t)3 * s] * P.tdims[(size_t)3 * s + 1] * P.tdims[(size_t)3 * s + 2];
+        tci_status st = n > 0 ? direct_tensor(b->ctx, R, s, n, h.data() + P.off[(size_t)5 * s]) : TCI_OK;
+        for (int w = 0; w < 4 && st == TCI_OK; ++w) {
+            const int cnt = P.counts[(size_t)w * R.L + s], len = set_len(R, w, s);
+            if (cnt && len) st = direct_set(b->ctx, R, w, s, cnt, len, h.data() + tb + P.off[(size_t)5 * s + 1 + w]);
         }
-        b->hostpacks.push_back(std::move(h));
-        P.T = (const double *)b->hostpacks.back().data();
-        P.sets = b->hostpacks.back().data() + tb;
-        b->packed[(size_t)i] = std::move(P);
-        return TCI_OK;
+        if (st != TCI_OK) return st;
     }
-    // the group to pack: i, and from the second solve on every other one left
+    b->hostpacks.push_back(std::move(h));
+    P.T = (const double *)b->hostpacks.back().data();
+    P.sets = b->hostpacks.back().data() + tb;
+    b->packed[(size_t)i] = std::move(P);
+    return TCI_OK;
+}
+
+constexpr size_t kPackGroupBytes = (size_t)1 << 30;
+constexpr size_t kPackGroupBlocks = (size_t)1 << 22;   // workgroups of a pack launch
+
+// Solve i's results packed on the device and downloaded, with up to `more` of those
+// that follow it (solves that ended for want of capacity apart, which a caller
+// submits again): at most what the context's HBM budget has left, which the packing
+// buffer is held against.  TCI_ERR_OOM: no room for it.
+static tci_status pack_group(tci_batch *b, int32_t i, const SolveDesc &R, int64_t more)
+{
+    tci_ctx *ctx = b->ctx;
+    const size_t left = ctx->budget > ctx->used ? (size_t)(ctx->budget - ctx->used) : 0;
+    const size_t room = std::min(left, kPackGroupBytes);
     std::vector<int32_t> solve(1, i);
     std::vector<tci_batch::Packed> P(1);
     std::vector<size_t> start(1, 0), tbs(1, 0);
-    size_t total = pack_shape(R, P[0], &tbs[0]);
+    size_t total = pack_shape(R, P[0], &tbs[0]), tb = 0;
     int L0 = R.L;
-    if (b->npacked > 0)
-        for (int32_t q = 0; q < b->count; ++q) {
-            if (q == i || !b->packed[(size_t)q].counts.empty()) continue;
-            SolveDesc Q;
-            if (!report_view(b, q, Q)) continue;
-            tci_batch::Packed p;
-            const size_t bytes = pack_shape(Q, p, &tb);
-            if (total + bytes > kPackGroupBytes) break;
-            solve.push_back(q);
-            P.push_back(std::move(p));
-            start.push_back(total);
-            tbs.push_back(tb);
-            total += bytes;
-            L0 = Q.L > L0 ? Q.L : L0;
-        }
-    const size_t n = solve.size();
-    if (n * (size_t)L0 > (size_t)INT32_MAX) return set_err(TCI_ERR_ARG, "too many solves");
+    // (a group's tables: an index per solve, five offsets per solve and site)
+    const auto tables = [](size_t n, int L) { return lay_align(4 * n) + lay_align(40 * n * (size_t)L) + 16; };
+    for (int32_t k = 1; k < b->count && more > 0; ++k) {
+        const int32_t q = (i + k) % b->count;
+        if (!b->packed[(size_t)q].counts.empty()) continue;
+        SolveDesc Q;
+        if (!report_view(b, q, Q) || !Q.ints[INT_DONE] || Q.ints[INT_STATUS] == TCI_ERR_CAPACITY) continue;
+        tci_batch::Packed p;
+        const size_t bytes = pack_shape(Q, p, &tb);
+        const int L1 = std::max(L0, (int)Q.L);
+        if (total + bytes + tables(solve.size() + 1, L1) > room || (solve.size() + 1) * (size_t)L1 > kPackGroupBlocks)
+            break;
+        solve.push_back(q);
+        P.push_back(std::move(p));
+        start.push_back(total);
+        tbs.push_back(tb);
+        total += bytes;
+        L0 = L1;
+        --more;
+    }
+    const size_t n = solve.size(), need = total + tables(n, L0);
+    if (need > left) return TCI_ERR_OOM;
     std::vector<int64_t> at(5 * n * (size_t)L0, 0);
     for (size_t q = 0; q < n; ++q)
         for (size_t s = 0; 5 * s < P[q].off.size(); ++s)
@@ -2031,21 +2057,28 @@ static tci_status ensure_packed(tci_batch *b, int32_t i)
     void *dev = nullptr;
     size_t got = 0;
     PoolBuf host{nullptr, 0};
-    hipError_t e = pool_get(ctx, b_idx + b_at + total + 16, &dev, &got);
-    if (e != hipSuccess) return set_err(TCI_ERR_OOM, "packed results: %s", hipGetErrorString(e));
+    ctx->used += need;   // (the pool makes room within the budget)
+    hipError_t e = pool_get(ctx, need, &dev, &got);
+    if (e == hipSuccess && (e = hpool_get(ctx, total + 16, &host)) != hipSuccess) pool_put(ctx, dev, got);
+    if (e != hipSuccess) {
+        ctx->used -= need;
+        (void)hipGetLastError();
+        return TCI_ERR_OOM;
+    }
     uint8_t *d = (uint8_t *)dev;
-    e = hpool_get(ctx, total + 16, &host);
-    if (e == hipSuccess) e = hipMemcpyAsync(d, solve.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, ctx->dl);
+    e = hipMemcpyAsync(d, solve.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, ctx->dl);
     if (e == hipSuccess)
         e = hipMemcpyAsync(d + b_idx, at.data(), sizeof(int64_t) * at.size(), hipMemcpyHostToDevice, ctx->dl);
     if (e == hipSuccess)
         e = launch_pack(b->d_desc, (const int32_t *)d, (int)n, L0, (const int64_t *)(d + b_idx), d + b_idx + b_at, ctx->dl);
     if (e == hipSuccess && total)
         e = hipMemcpyAsync(host.ptr, d + b_idx + b_at, total, hipMemcpyDeviceToHost, ctx->dl);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->dl);
+    const hipError_t es = hipStreamSynchronize(ctx->dl);
+    if (e == hipSuccess) e = es;
+    ctx->used -= need;
     pool_put(ctx, dev, got);
     if (e != hipSuccess) {
-        if (host.ptr) hpool_put(ctx, host);
+        hpool_put(ctx, host);
         return set_err(TCI_ERR_DEVICE, "packed results: %s", hipGetErrorString(e));
     }
     b->packs.push_back(host);
@@ -2058,6 +2091,34 @@ static tci_status ensure_packed(tci_batch *b, int32_t i)
     return TCI_OK;
 }
 
+// Solve i's site tensors and index sets in host memory.  A solve is packed with up
+// to three others for each one packed before it, so that a batch that is read whole
+// takes a few downloads (one per tensor and set costs 25 us each, and a batch of 384
+// solves has 15 000 of them: 640 ms against 3 for the solves themselves), and never
+// more than four times the solves asked for are kept.  Where there is no room to
+// pack, and for a served request, whose pack kernel could have to wait for the
+// resident grid, the pieces are read one by one.
+static tci_status ensure_packed(tci_batch *b, int32_t i)
+{
+    SolveDesc R;
+    if (!report_view(b, i, R)) return set_err(TCI_ERR_ARG, "bad batch/index");
+    if (b->packed.empty()) b->packed.resize((size_t)b->count);
+    if (!b->packed[(size_t)i].counts.empty()) return TCI_OK;
+    HIPCHK(hipSetDevice(b->ctx->device));
+    if (!b->served) {
+        tci_status s = pack_group(b, i, R, 3 * (int64_t)b->npacked);
+        if (s == TCI_ERR_OOM && b->npacked > 0) s = pack_group(b, i, R, 0);
+        if (s != TCI_ERR_OOM) return s;
+    }
+    return direct_solution(b, i, R);
+}
+
+// a served request's results not read yet: its accessors read what they are asked for
+static bool read_direct(const tci_batch *b, int32_t i)
+{
+    return b->served && (b->packed.empty() || b->packed[(size_t)i].counts.empty());
+}
+
 tci_status tci_batch_indexset(tci_batch *b, int32_t i, int32_t which, int32_t site, int32_t *count,
                               uint8_t *out, int64_t cap_bytes)
 {
@@ -2068,6 +2129,7 @@ tci_status tci_batch_indexset(tci_batch *b, int32_t i, int32_t which, int32_t si
     *count = n;
     if ((int64_t)n * len > cap_bytes || (!out && n * len > 0)) return set_err(TCI_ERR_ARG, "output buffer too small");
     if (n == 0 || len == 0) return TCI_OK;
+    if (read_direct(b, i)) return direct_set(b->ctx, R, which, b0, n, len, out);
     const tci_status s = ensure_packed(b, i);
     if (s != TCI_OK) return s;
     const tci_batch::Packed &P = b->packed[(size_t)i];
@@ -2083,6 +2145,7 @@ tci_status tci_batch_sitetensor(tci_batch *b, int32_t i, int32_t site, int64_t *
     const int64_t n = dims3[0] * dims3[1] * dims3[2];
     if (n > cap || (!out && n > 0)) return set_err(TCI_ERR_ARG, "output buffer too small");
     if (n == 0) return TCI_OK;
+    if (read_direct(b, i)) return direct_tensor(b->ctx, R, site - 1, n, out);
     const tci_status s = ensure_packed(b, i);
     if (s != TCI_OK) return s;
     const tci_batch::Packed &P = b->packed[(size_t)i];
