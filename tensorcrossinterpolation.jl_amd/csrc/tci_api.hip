@@ -71,6 +71,7 @@ struct tci_ctx {
     std::vector<PoolBuf> pool;          // cached device buffers of finished batches
     std::vector<PoolBuf> hpool;         // cached pinned buffers of packed results
     uint64_t pooled = 0;                // their bytes
+    std::vector<std::vector<uint8_t>> spare;   // host staging of finished batches
     int lds_wg;         // LDS bytes (static + dynamic) a solve workgroup of the default team may use
     int team;           // threads per solve workgroup (the default team)
     bool team_env = false;   // set by TCI_TEAM
@@ -230,6 +231,35 @@ static void hpool_put(tci_ctx *c, const PoolBuf &b)
     for (const PoolBuf &q : c->hpool) tot += q.bytes;
     if (!b.pinned || tot > kHostPoolBytes || c->hpool.size() >= kHostPoolBufs) host_free(b);
     else c->hpool.push_back(b);
+}
+
+// Host staging (input images and reports) kept between batches: up to
+// kSpareBytes in at most kSpareBufs vectors.  Given back to the allocator and taken
+// again, the 14 MB of 4096 solves are unmapped and mapped anew each time, as they are
+// more than glibc keeps at the heap's end: 1.4 ms for a submit that takes 0.5.
+constexpr size_t kSpareBytes = (size_t)64 << 20;
+constexpr size_t kSpareBufs = 8;
+
+// a vector of `bytes` bytes, whose contents are whatever they were
+static std::vector<uint8_t> spare_get(tci_ctx *c, size_t bytes)
+{
+    std::vector<uint8_t> v;
+    for (size_t i = 0; i < c->spare.size(); ++i)
+        if (c->spare[i].capacity() >= bytes && c->spare[i].capacity() <= 4 * bytes + (1 << 20)) {
+            v.swap(c->spare[i]);
+            c->spare.erase(c->spare.begin() + (long)i);
+            break;
+        }
+    v.resize(bytes);
+    return v;
+}
+
+static void spare_put(tci_ctx *c, std::vector<uint8_t> &v)
+{
+    size_t tot = v.capacity();
+    if (tot < ((size_t)128 << 10)) return;   // (small ones never leave the heap)
+    for (const auto &q : c->spare) tot += q.capacity();
+    if (tot <= kSpareBytes && c->spare.size() < kSpareBufs) c->spare.push_back(std::move(v));
 }
 
 // a block of a slot-level server's memory: device memory, or pinned host
@@ -1629,6 +1659,10 @@ static void batch_release(tci_batch *b)
     }
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
+    if (b->ctx) {
+        spare_put(b->ctx, b->h_in);
+        spare_put(b->ctx, b->h_rep);
+    }
     for (const PoolBuf &q : b->packs) {
         if (b->ctx) hpool_put(b->ctx, q);
         else host_free(q);
@@ -1709,7 +1743,8 @@ static tci_status batch_prepare(tci_ctx *ctx, int32_t count, const tci_problem *
     b->rep_bytes = trep;
     b->desc.resize((size_t)count);
     b->rep_off.resize((size_t)count);
-    b->h_in.assign(tin, 0);
+    b->h_in = spare_get(ctx, tin);
+    memset(b->h_in.data(), 0, tin);
     uint8_t *himg = b->h_in.data();
     size_t oin = 0, ost = 0, orp = 0;
     for (int i = 0; i < count; ++i) {
@@ -1836,7 +1871,7 @@ static tci_status fetch_reports(tci_batch *b)
 {
     if (b->fetched) return TCI_OK;
     HIPCHK(hipSetDevice(b->ctx->device));
-    b->h_rep.resize(b->rep_bytes);
+    if (b->h_rep.size() != b->rep_bytes) b->h_rep = spare_get(b->ctx, b->rep_bytes);
     if (b->served) {
         // poll the done mark (relaunching the grid if it went idle); the
         // workgroup copied the report to pinned host memory before it
