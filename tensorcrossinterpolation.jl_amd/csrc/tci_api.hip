@@ -647,6 +647,7 @@ static tci_status lu_partition(tci_ctx *ctx, int64_t tile_budget, LuPlan &P, boo
 
 // One launch of an on-chip kernel over its jobs: the largest teams first, and
 // among equal teams the largest matrices, so the launch ends on small ones.
+// TCI_ERR_OOM, with nothing launched, when there is no memory for their scratch.
 static tci_status lu_run_chip(tci_ctx *ctx, tci_lu_job *jobs, const LuPlan &P, std::vector<ChipItem> items, int big)
 {
     if (items.empty()) return TCI_OK;
@@ -678,7 +679,10 @@ static tci_status lu_run_chip(tci_ctx *ctx, tci_lu_job *jobs, const LuPlan &P, s
     for (size_t q = 0; q < items.size(); ++q)
         for (int32_t g = 0; g < items[q].S; ++g) *map++ = (int32_t)q;
     uint8_t *d = nullptr;
-    HIPCHK(hipMallocAsync((void **)&d, b_items + b_map + b_mail + b_cols + b_spill, st));
+    if (hipMallocAsync((void **)&d, b_items + b_map + b_mail + b_cols + b_spill, st) != hipSuccess) {
+        (void)hipGetLastError();
+        return TCI_ERR_OOM;
+    }
     hipError_t e = hipMemcpyAsync(d, h.data(), b_items + b_map, hipMemcpyHostToDevice, st);
     uint8_t *z = d + b_items + b_map;
     if (e == hipSuccess) e = hipMemsetAsync(z, 0, b_mail, st);
@@ -736,11 +740,14 @@ static tci_status lu_launch(tci_ctx *ctx, tci_lu_job *jobs, LuPlan &P)
     if (ps != TCI_OK) return ps;
     std::vector<int32_t> &tile = P.tile, &stream = P.stream;
     if (ctx->lu_queued) HIPCHK(lu_wait(ctx));
-    ps = lu_run_chip(ctx, jobs, P, P.chip, 0);
-    if (ps != TCI_OK) return ps;
-    if (!P.chip.empty() && !P.big.empty()) HIPCHK(lu_wait(ctx));   // (chip_host is used again)
-    ps = lu_run_chip(ctx, jobs, P, P.big, 1);
-    if (ps != TCI_OK) return ps;
+    for (int big = 0; big < 2; ++big) {
+        const std::vector<ChipItem> &items = big ? P.big : P.chip;
+        if (big && !items.empty() && !P.chip.empty()) HIPCHK(lu_wait(ctx));   // (chip_host is used again)
+        ps = lu_run_chip(ctx, jobs, P, items, big);
+        if (ps == TCI_ERR_OOM)   // streamed instead
+            for (const ChipItem &it : items) stream.push_back(it.job);
+        else if (ps != TCI_OK) return ps;
+    }
     if (!tile.empty()) {
         uint8_t *d = nullptr;
         const size_t b_idx = lay_align(sizeof(int32_t) * tile.size());
@@ -2337,31 +2344,41 @@ static tci_status tt_eval_device(tci_ctx *ctx, hipStream_t st, int L, const std:
                                  const int32_t *d_iparams, double *tt_out, double *f_out, double *maxerr,
                                  double *maxabsf)
 {
-    const bool grouped = tt_grouped(npts, L, dims3, chimax);
-    int64_t chunk = npts, dmax = 1;
-    if (grouped) {
-        chunk = std::max((int64_t)64, (int64_t)(kTtVecBytes / (16 * (size_t)chimax)) & ~(int64_t)255);
-        chunk = std::min(npts, chunk);
-        for (int b = 0; b < L; ++b) dmax = std::max(dmax, dims3[(size_t)(3 * b + 1)]);
-    }
-    const int np = grouped ? 256 : tt_eval_points_per_block(chimax);
-    const int64_t blocks = (npts + np - 1) / np;
-    const int64_t maxtiles = chunk / 64 + dmax + 1;
-    if (grouped && maxtiles > INT32_MAX) return set_err(TCI_ERR_ARG, "too many points");
-    size_t need = 0;
-    auto a = [&](size_t bytes) { size_t at = need; need = lay_align(need + (bytes ? bytes : 1)); return at; };
-    const size_t o_pts = a((size_t)(npts * L));
-    const size_t o_tt = a(sizeof(double) * (size_t)npts);
-    const size_t o_f = a(sizeof(double) * (size_t)npts);
-    const size_t o_bm = a(sizeof(double) * (size_t)(2 * blocks));
-    const size_t o_bins = a(grouped ? sizeof(int32_t) * 256 * (size_t)L : 0);
-    const size_t o_nt = a(grouped ? sizeof(int32_t) * (size_t)L : 0);
-    const size_t o_tiles = a(grouped ? sizeof(TtTile) * (size_t)maxtiles * (size_t)L : 0);
-    const size_t o_ord = a(grouped ? sizeof(int32_t) * (size_t)chunk * (size_t)L : 0);
-    const size_t o_v = a(grouped ? sizeof(double) * (size_t)chunk * (size_t)chimax : 0);
-    const size_t o_w = a(grouped ? sizeof(double) * (size_t)chunk * (size_t)chimax : 0);
+    bool grouped = tt_grouped(npts, L, dims3, chimax);
+    int64_t chunk, dmax, blocks, maxtiles;
+    size_t need, o_pts, o_tt, o_f, o_bm, o_bins, o_nt, o_tiles, o_ord, o_v, o_w;
     uint8_t *d = nullptr;
-    HIPCHK(hipMallocAsync((void **)&d, need, st));
+    for (;;) {
+        chunk = npts;
+        dmax = 1;
+        if (grouped) {
+            chunk = std::max((int64_t)64, (int64_t)(kTtVecBytes / (16 * (size_t)chimax)) & ~(int64_t)255);
+            chunk = std::min(npts, chunk);
+            for (int b = 0; b < L; ++b) dmax = std::max(dmax, dims3[(size_t)(3 * b + 1)]);
+        }
+        const int np = grouped ? 256 : tt_eval_points_per_block(chimax);
+        blocks = (npts + np - 1) / np;
+        maxtiles = chunk / 64 + dmax + 1;
+        if (grouped && maxtiles > INT32_MAX) return set_err(TCI_ERR_ARG, "too many points");
+        need = 0;
+        auto a = [&](size_t bytes) { size_t at = need; need = lay_align(need + (bytes ? bytes : 1)); return at; };
+        o_pts = a((size_t)(npts * L));
+        o_tt = a(sizeof(double) * (size_t)npts);
+        o_f = a(sizeof(double) * (size_t)npts);
+        o_bm = a(sizeof(double) * (size_t)(2 * blocks));
+        o_bins = a(grouped ? sizeof(int32_t) * 256 * (size_t)L : 0);
+        o_nt = a(grouped ? sizeof(int32_t) * (size_t)L : 0);
+        o_tiles = a(grouped ? sizeof(TtTile) * (size_t)maxtiles * (size_t)L : 0);
+        o_ord = a(grouped ? sizeof(int32_t) * (size_t)chunk * (size_t)L : 0);
+        o_v = a(grouped ? sizeof(double) * (size_t)chunk * (size_t)chimax : 0);
+        o_w = a(grouped ? sizeof(double) * (size_t)chunk * (size_t)chimax : 0);
+        const hipError_t em = hipMallocAsync((void **)&d, need, st);
+        if (em == hipSuccess) break;
+        if (!grouped) return set_err(TCI_ERR_DEVICE, "TT evaluation: %s", hipGetErrorString(em));
+        // no memory for the running vectors of a chunk: the route without them
+        (void)hipGetLastError();
+        grouped = false;
+    }
     hipError_t e = hipMemcpyAsync(d + o_pts, pts, (size_t)(npts * L), hipMemcpyHostToDevice, st);
     if (!grouped && e == hipSuccess)
         e = launch_tt_eval(L, d_dims3, d_coff, d_cores, d + o_pts, npts, chimax, fkind, d_params, d_iparams,
