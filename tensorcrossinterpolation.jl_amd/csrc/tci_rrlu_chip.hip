@@ -56,7 +56,7 @@
 // update and 3.5 the three dependent round trips between XCDs (column stores
 // acknowledged, mailbox seen, winner's column read); the big kernel adds the
 // streaming of the columns in memory, at about 6 TB/s.  1024 matrices of 32 to
-// 1024 rows and columns, rank 8 to 128: 118.5 -> 20.6 ms a pass against the
+// 1024 rows and columns, rank 8 to 128: 118.2 -> 20.0 ms a pass against the
 // streaming kernel (one workgroup per matrix, 16 B per entry and pivot); one
 // 1024 x 1024 matrix of rank 64: 2.3 -> 0.55 ms, one 4352 x 4352 with 256
 // pivots: 21.8 -> 7.2 ms against a grid-wide kernel that streamed the matrix
@@ -733,7 +733,7 @@ __device__ __forceinline__ void chip_failed(const ChipArgs &K, int ticket)
 }
 
 // the register shapes, by ChipItem::shape: rows per lane × columns per wave.
-// 80 to 85 entries a thread: with the pivot column, positions and addresses
+// 72 to 88 entries a thread: with the pivot column, positions and addresses
 // that fills 256 registers without spilling
 __global__ __launch_bounds__(256, 2) void tci_rrlu_chip_kernel(ChipArgs K)
 {
@@ -758,6 +758,8 @@ __global__ __launch_bounds__(256, 2) void tci_rrlu_chip_kernel(ChipArgs K)
     }
 }
 
+// (the columns outside the registers cost some more: 121 values in 212 bytes of
+// scratch over the four shapes)
 __global__ __launch_bounds__(512, 2) void tci_rrlu_chip_big_kernel(ChipArgs K, int64_t exl_cap)
 {
     __shared__ ChipLds<8> sh;
